@@ -1,33 +1,28 @@
-// fp32 GEMM on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32).
+// fp32 GEMM on the gfx950 matrix cores.
 //
 // Replaces cublasSgemm / cublasSgemmStridedBatched behind ops::matmul and
-// ops::bmm (reference src/ops/matmul.cpp:13-93).  Kernel templates cover the
-// four transpose cases: each operand tile is K-contiguous (read as b128, one
-// LDS read feeds four MFMA k-steps) or MN-contiguous (read as b32 with
-// consecutive lanes on consecutive rows).  The k index an MFMA step consumes
-// is permuted so that lane group g = lane/32 owns k = 8*slab + 4*g + j for
-// step j; A and B use the same permutation, so the contraction is unchanged.
+// ops::bmm (reference src/ops/matmul.cpp:13-93).  Each operand is K-contiguous
+// or MN-contiguous, which covers the four transpose cases.
 //
-// Block tiles 128x128 (three blocks per CU) or 256x128 (two per CU), 256
-// threads = 4 waves in 2x2, wave tile (BM/2)x(BN/2) of 32x32 MFMA tiles held
-// in accumulation registers.  A stage is BK = 16 = two k slabs, software
-// pipelined inside one wave so the matrix core never waits on LDS (ordering
-// fixed with sched_group_barrier): slab-0 MFMAs under the LDS reads of slab 1,
-// one barrier, the next stage's slab-0 reads under the last slab-1 MFMAs.
+// Main path, gemm_f32_split: every fp32 value is split, exactly, into three
+// bf16 values on its way to LDS, and a product is six bf16 MFMAs into fp32
+// accumulators: 2.5 PFLOP/s / 6 = 0.42 PFLOP/s where the fp32 MFMAs have
+// 0.157.  Against 64-bit sums its error is 0.85 of theirs (see the kernel).
 //
-// Main path, gemm_f32_dma: tiles are copied global -> LDS by
-// global_load_lds_dwordx4 (no register staging, no LDS store instructions)
-// into a 3-stage ring, two stages ahead of the MFMAs, with swizzled layouts
-// instead of padding.  Fallback, gemm_f32_mfma (K % 16 != 0, unaligned or
-// odd-width operands): global -> registers -> LDS, double-buffered, the
-// stores interleaved with the MFMAs.  Both accumulate in the same k order,
-// so they give identical bits.
+// Fallback, gemm_f32_mfma (rows that are not whole aligned float4s, offsets
+// past 2 GB): v_mfma_f32_32x32x2_f32, tiles 128x128 (three blocks per CU) or
+// 256x128 (two), 256 threads = 4 waves in 2x2, a stage of BK = 16 k = two
+// slabs of 8: global -> registers -> LDS, double-buffered, pipelined inside
+// one wave so the matrix core never waits on LDS (ordering fixed with
+// sched_group_barrier).  The k index an MFMA step consumes is permuted so
+// that lane group g = lane/32 owns k = 8*slab + 4*g + j for step j; A and B
+// use the same permutation, so the contraction is unchanged.
 //
 // Tiles are ordered so that tiles sharing A rows land on the same XCD (block
 // b runs on XCD b % 8) and, within it, in groups of 8 tile rows for L2 reuse.
-// Small output grids with a long K (weight gradients: M, N = features,
-// K = tokens) are split along K into a workspace of partial products that a
-// second kernel sums in a fixed order, so results stay bitwise reproducible.
+// Small output grids are split along K into a workspace of partial products
+// that a second kernel sums in a fixed order, so results stay bitwise
+// reproducible.
 #include <type_traits>
 
 #include "common.h"
@@ -52,8 +47,7 @@ struct GemmArgs {
   int64_t kchunk;  // > 0: blockIdx.y is a K split of this many k (last one clipped)
   float alpha, beta;
   int tiles_m, tiles_n;
-  // Optional extent read from device memory at run time (LDS-DMA kernel and
-  // the split-K reduce only): v = clamp(*dyn - dyn_base, 0, static extent);
+  // Optional extent read from device memory at run time: v = clamp(*dyn - dyn_base, 0, static extent);
   // dyn_dim 0: rows of C beyond v are not needed (whole tiles past v exit);
   // dyn_dim 1: K becomes v rounded up to 16 (operand rows up to there are read).
   const int64_t* dyn = nullptr;
@@ -197,9 +191,17 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_mfma(GemmArgs a) {
   const float* __restrict__ A = a.A + bz * a.sA;
   const float* __restrict__ B = a.B + bz * a.sB;
   float* __restrict__ C = a.C + bz * a.sC;
-  const int64_t K = a.kchunk > 0 ? min(a.kchunk, a.K - bz * a.kchunk) : a.K;
+  int64_t K = a.kchunk > 0 ? min(a.kchunk, a.K - bz * a.kchunk) : a.K;
   const int64_t m0 = static_cast<int64_t>(tm) * BM;
   const int64_t n0 = static_cast<int64_t>(tn) * BN;
+  if (a.dyn) {  // uniform per block: the whole block leaves or none of it
+    if (a.dyn_dim == 0) {
+      if (m0 >= dyn_extent(a, a.M)) return;
+    } else {
+      K = min(K, (dyn_extent(a, K) + 15) / 16 * 16);
+      if (K == 0 && a.beta == 1.f && !a.D) return;  // C stays as it is
+    }
+  }
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -304,112 +306,199 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_mfma(GemmArgs a) {
 }
 
 
-// ---------------------------------------------------------------- LDS DMA
-// Operand tiles go global -> LDS with global_load_lds_dwordx4: lane L of a
-// wave-instruction writes 16 bytes at LDS base + 16 L, so one instruction
-// fills a contiguous 1 KB block and the choice of which global 16 bytes each
-// lane fetches sets the layout.  No registers stage the tile and no LDS store
-// instruction runs.
-//   K-contiguous tile [ROWS][16]: 16-row blocks of 64 16-byte units; row x's
-//     k-chunk c sits at unit 4 (x % 16) + (c ^ swz(x % 16)).
-//   MN-contiguous tile [16][ROWS]: k-row k's chunk q (4 floats) sits at
-//     chunk position q ^ (8 ((k >> 2) & 1)).
-// Both keep the fragment reads free of bank conflicts without padding.
-__device__ __forceinline__ int swz(int x) { return ((x >> 1) ^ (x >> 3)) & 3; }
+// ------------------------------------------------- bf16 matrix cores, fp32 in
+// Every fp32 value is the sum of three bf16 values exactly (8 + 8 + 8
+// significand bits, each part rounded to nearest): x = x0 + x1 + x2.  A
+// product is then taken as the six partial products
+//   a0 b2 + a1 b1 + a2 b0 + a0 b1 + a1 b0 + a0 b0
+// on v_mfma_f32_32x32x16_bf16, whose products are exact and whose sums are
+// fp32; what is left out (a1 b2, a2 b1, a2 b2) is below 2^-26 of the product.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-//   BUF: the copies are buffer_load_dwordx4 ... lds through a buffer resource
-//     based at the block's first row (K-contiguous) or column (MN-contiguous),
-//     with 32-bit per-lane byte offsets and the stage's offset in an SGPR;
-//     otherwise global_load_lds_dwordx4 with a 64-bit address per lane.  Same
-//     bytes to the same LDS places: 1.3-2.1% faster on the c5 NT shapes (fewer
-//     address registers and address operations per copy).  The launcher picks
-//     BUF when every offset of the product stays below 2^31 bytes.
-template <bool KC, int ROWS, bool BUF>
-struct DmaTile {
-  static constexpr int kFloats = ROWS * 16;   // one stage
-  static constexpr int kInsts = ROWS / 64;    // wave-instructions per wave per stage
-  const float* src[kInsts];                    // !BUF: this lane's 16 bytes, stage 0
-  int64_t step;                                // !BUF: element stride between stages
-  __amdgpu_buffer_rsrc_t rsrc;                 // BUF: the block's first row / column
-  int voff[kInsts];                            // BUF: this lane's byte offset, stage 0
-  int bstep;                                   // BUF: bytes between stages
+__device__ __forceinline__ unsigned pack_bf16(float x, float y) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x, y}, bf16x2));
+}
+__device__ __forceinline__ float bf16_lo(unsigned u) { return __builtin_bit_cast(float, u << 16); }
+__device__ __forceinline__ float bf16_hi(unsigned u) {
+  return __builtin_bit_cast(float, u & 0xffff0000u);
+}
 
-  __device__ __forceinline__ void init(const float* X, int64_t ld, int64_t R, int64_t row0,
-                                       int w, int lane) {
-    const int64_t base = KC ? row0 * ld : row0;  // elements from X to the buffer's start
-    if constexpr (BUF)
-      rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(X + base), 0, 0x7fffffff,
-                                               0x00020000);
+struct SplitWork {  // four k of one row on their way from fp32 to three parts
+  float x[4];
+  u32x2 part[3];
+};
+
+// One operand's tile: ROWS rows x 16 k of fp32, fetched into registers and
+// stored to LDS as three bf16 planes of [2 k halves][ROWS slots][8 k].  An
+// MFMA fragment (32 slots, one k half per lane group) is then one b128 read
+// of 512 contiguous bytes per half; the halves lie 128 bytes apart modulo the
+// 64 banks, so that the stores of four k per lane meet no bank twice.
+//   K-contiguous: lane = (row, k quad), slot = row.
+//   MN-contiguous: a wave takes one k quad; a lane takes P = ROWS / 64
+//     consecutive rows of each of its four k, and row P l + i goes to slot
+//     32 P (l / 32) + 32 i + l % 32, so that a lane's rows land in the P
+//     32-slot tiles of one wave at the same place.
+template <bool KC, int ROWS>
+struct SplitTile {
+  static constexpr int P = ROWS / 64;
+  static constexpr int kHalf = ROWS * 16 + 128;   // bytes
+  static constexpr int kPlane = 2 * kHalf;
+  static constexpr int kBytes = 3 * kPlane;
+  const char* base;      // the tile's first element at the current stage
+  int64_t left;          // bytes from there to the operand's end
+  int64_t step;          // bytes between stages
+  int voff;              // this lane's first element, bytes from base
+  int soff[KC ? P : 4];  // uniform offsets of the lane's loads
+  int woff;              // where the lane's first four k go in LDS
+  using Vec = std::conditional_t<KC || P == 4, f32x4, f32x2>;
+  Vec reg[KC ? P : 4];   // K-contiguous: four k of a row; MN: P rows of a k
+
+  __device__ __forceinline__ void init(const float* X, int64_t ld, int64_t R, int64_t K,
+                                       int64_t row0, int wave, int lane) {
+    if constexpr (KC) {
+      base = reinterpret_cast<const char*>(X + row0 * ld);
+      left = ((R - row0 - 1) * ld + K) * 4;
+      step = 64;
+      const int row = 16 * wave + (lane >> 2), quad = lane & 3;
+      voff = static_cast<int>(row * ld * 4) + 16 * quad;
 #pragma unroll
-    for (int q = 0; q < kInsts; ++q) {
-      const int t = w + 4 * q;  // 1 KB block of the tile
-      int64_t e;                // this lane's first element
-      if (KC) {
-        const int x = lane >> 2;
-        const int64_t row = min(row0 + 16 * t + x, R - 1);  // rows past R: never stored
-        e = row * ld + 4 * ((lane & 3) ^ swz(x));
-      } else {
-        constexpr int kRowsPer = 256 / ROWS;   // k-rows per 1 KB block
-        constexpr int kLanesPer = 64 / kRowsPer;
-        const int k = t * kRowsPer + lane / kLanesPer;
-        const int q4 = (lane % kLanesPer) ^ (8 * ((k >> 2) & 1));
-        const int64_t col = min(row0 + 4 * q4, R - 4);      // R % 4 == 0 on this path
-        e = k * ld + col;
-      }
-      if constexpr (BUF)
-        voff[q] = static_cast<int>((e - base) * 4);
-      else
-        src[q] = X + e;
+      for (int q = 0; q < P; ++q) soff[q] = static_cast<int>(q * 64 * ld * 4);
+      woff = (quad >> 1) * kHalf + row * 16 + (quad & 1) * 8;
+    } else {
+      base = reinterpret_cast<const char*>(X + row0);
+      left = ((K - 1) * ld + R - row0) * 4;
+      step = 64 * ld;
+      voff = 4 * P * lane;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) soff[j] = static_cast<int>((4 * wave + j) * ld * 4);
+      woff = (wave >> 1) * kHalf + (32 * P * (lane >> 5) + (lane & 31)) * 16 + (wave & 1) * 8;
     }
-    step = KC ? 16 : 16 * ld;
-    bstep = static_cast<int>(4 * step);
   }
-  // Stage kt of this lane's loads into the stage buffer `dst` (LDS).
-  __device__ __forceinline__ void issue(float* dst, int64_t kt, int w) const {
-#if defined(__HIP_DEVICE_COMPILE__)  // the host pass would drop the kernel's launch stub
-#pragma unroll
-    for (int q = 0; q < kInsts; ++q) {
-      float* d = dst + 256 * (w + 4 * q);
-      if constexpr (BUF)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rsrc, (__attribute__((address_space(3))) void*)d, 16, voff[q],
-            static_cast<int>(kt) * bstep, 0, 0);
-      else
-        __builtin_amdgcn_global_load_lds(src[q] + kt * step, d, 16, 0, 0);
-    }
+
+  static constexpr int kLoads = KC ? P : 4;
+  // Load q of the current stage.  Past the operand's end the buffer resource
+  // returns zeros, so no row or k is tested, except k past K in a
+  // K-contiguous row (`at`).
+  __device__ __forceinline__ void load(int q) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(base), 0, static_cast<int>(min(max(left, int64_t{0}), int64_t{0x7fffffff})),
+        0x00020000);
+    if constexpr (sizeof(Vec) == 16)
+      reg[q] =
+          __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b128(rs, voff + soff[q], 0, 0));
+    else
+      reg[q] =
+          __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b64(rs, voff + soff[q], 0, 0));
 #endif
+  }
+  __device__ __forceinline__ void next() {
+    base += step;
+    left -= step;
+  }
+  __device__ __forceinline__ void load_all() {
+#pragma unroll
+    for (int q = 0; q < kLoads; ++q) load(q);
+    next();
+  }
+  // Element (k j of the lane's quad, row i of the lane's P).
+  __device__ __forceinline__ float at(int j, int i) const {
+    return KC ? reg[i][j] : reg[j][i];
+  }
+  // The split of row i's four k, in kSteps steps of at most four VALU
+  // operations for the spaces between MFMAs; the last stores the parts.
+  // MASK: a K-contiguous lane's k count only when `valid`.  FLIP: `sign` (0 or the sign
+  // bit) is applied first.
+  static constexpr int kSteps = 7;
+  template <bool FLIP, bool MASK>
+  __device__ __forceinline__ void split_step(SplitWork& w, int i, int step, char* lds, bool valid,
+                                             unsigned sign) const {
+    if (step == 0 || step == 3) {
+      if (step == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float v = MASK && KC && !valid ? 0.f : at(j, i);
+          w.x[j] = FLIP ? __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ sign) : v;
+        }
+      }
+      const int p = step / 3;
+      w.part[p] = u32x2{pack_bf16(w.x[0], w.x[1]), pack_bf16(w.x[2], w.x[3])};
+    } else if (step == 2 || step == 5) {
+      const u32x2 h = w.part[step / 3];
+      w.x[0] -= bf16_lo(h[0]);
+      w.x[1] -= bf16_hi(h[0]);
+      w.x[2] -= bf16_lo(h[1]);
+      w.x[3] -= bf16_hi(h[1]);
+    } else if (step == 6) {
+      w.part[2] = u32x2{pack_bf16(w.x[0], w.x[1]), pack_bf16(w.x[2], w.x[3])};
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<u32x2*>(lds + woff + p * kPlane + i * (KC ? 64 : 32) * 16) = w.part[p];
+    }
+  }
+  template <bool FLIP, bool MASK>
+  __device__ __forceinline__ void store_all(char* lds, bool valid, unsigned sign) const {
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      SplitWork w;
+#pragma unroll
+      for (int t = 0; t < kSteps; ++t) split_step<FLIP, MASK>(w, i, t, lds, valid, sign);
+    }
+  }
+  // Part p of 32-slot tile t (from the wave's first), for lane offset `off`.
+  __device__ __forceinline__ static bf16x8 frag(const char* lds, int off, int p, int t) {
+    return __builtin_bit_cast(bf16x8,
+                              *reinterpret_cast<const u32x4*>(lds + off + p * kPlane + t * 512));
   }
 };
 
-// Fragment of 32-row tile `i` for MFMA steps j = 0..3 of slab s: one b128
-// read at the lane's precomputed offset (K-contiguous), or four b32 reads of
-// k-rows 8 s + 4 g + j at column position ((mb4 + 8 i) ^ 8 g) * 4 + r
-// (MN-contiguous; mb4 = the wave's first column / 4).
-template <bool KC, int ROWS>
-__device__ __forceinline__ f32x4 dma_frag(const float* st, int off, int i, int s, int g, int r,
-                                          int mb4) {
-  if (KC) return *reinterpret_cast<const f32x4*>(st + off + i * 32 * 16);
-  f32x4 v;
-  const int q = (mb4 + 8 * i) ^ (8 * g);
-  const float* p = st + (8 * s + 4 * g) * ROWS + (q << 2) + r;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) v[j] = p[j * ROWS];
-  return v;
+// Why: the fp32 MFMAs reach 151 TFLOP/s (0.96 of their peak) and bound every
+// large product.  Here 32768x6144x2048 (NT) takes 3.42 ms against 5.48, 241
+// TFLOP/s: matrix cores 75% busy while power holds the clock near 1.9 GHz (on
+// zeros, which cost little power, the same launch takes 2.64 ms).
+// Error against 64-bit sums, normal data, K = 256 / 2048 / 32768: 2.4e-7,
+// 7.0e-7, 3.0e-6 in the 2-norm, where fp32 MFMAs give 2.9e-7, 8.1e-7, 3.2e-6.
+//
+// The bf16 MFMAs round their sums very slightly downwards (a mean of -1.3e-7
+// of the mean magnitude at K = 2048, in proportion to the number of sums and
+// their size), which sums over rows, columns or K splits would gather: with
+// it, a value projection's weight gradient over 32768 tokens was 1.4 times as
+// far from 64-bit sums as with fp32 MFMAs.  So the sum is held negated, B's
+// sign flipped on the way to LDS, from 0.207 to 0.707 of K, which cancels the
+// bias of sums that stay the same size along K or grow as sqrt(K), and all
+// but 9% where they grow as K (nothing here depends on a row's or column's
+// place).  K splits start negated by the parity of the number's count of ones
+// (0 1 1 0 1 0 0 1 ...).  Turning 256 accumulators costs about one stage.
+//
+// What the split cannot give: a value that is not finite, or beyond bf16's
+// range, has no three parts (the result is then not finite), and below 2^-110
+// the last part runs out of exponent.  Such a result, not finite or below
+// 2^-100, is found here and taken again in fp32.
+// `out_of_range` of a value's bits: at least kOutOfRange for such a value and
+// for a zero, which is told apart only when one of these is there.
+constexpr unsigned kSmall = 0x0d800000u, kInf = 0x7f800000u;  // 2^-100, infinity
+constexpr unsigned kOutOfRange = 2 * (kInf - kSmall);
+__device__ __forceinline__ unsigned out_of_range(unsigned bits) {
+  return (bits << 1) + (0u - 2 * kSmall);
 }
 
-template <bool A_KC, bool B_KC, int BM, int BN, int OCC, bool BUF>
-__global__ __launch_bounds__(kThreads, OCC) void gemm_f32_dma(GemmArgs a) {
-  using TA = DmaTile<A_KC, BM, BUF>;
-  using TB = DmaTile<B_KC, BN, BUF>;
+// 256 threads = 4 waves in 2x2, wave tiles (BM/2)x(BN/2); LDS is double
+// buffered.  A 256x256 block has a CU to itself and one wave per SIMD, so the
+// order of the wave's own instructions is what keeps the matrix core busy:
+// it is written out MFMA by MFMA and pinned (sched_barrier), two to eight
+// VALU operations of the split between two MFMAs of 32 cycles each.  Left to
+// the compiler, the same work ran at 207 TFLOP/s instead of 241.
+template <bool A_KC, bool B_KC, int BM, int BN, int OCC, bool TAIL>
+__global__ __launch_bounds__(kThreads, OCC) void gemm_f32_split(GemmArgs a) {
+  using TA = SplitTile<A_KC, BM>;
+  using TB = SplitTile<B_KC, BN>;
   constexpr int FI = BM / 64, FJ = BN / 64;
-  // An M-contiguous A on 256-row tiles is read as b128 rows of four
-  // consecutive tile rows (see load_a), one read per MFMA k-step of a slab.
-  constexpr bool kPermA = !A_KC && FI == 4;
-  constexpr int NR = (A_KC ? FI : kPermA ? 4 : 4 * FI) + FJ * (B_KC ? 1 : 4);
-  constexpr int NM = 4 * FI * FJ;
-  constexpr int kStage = TA::kFloats + TB::kFloats;
-  __shared__ __attribute__((aligned(1024))) float lds[3 * kStage];  // 3-stage ring
-  constexpr int NI = TA::kInsts + TB::kInsts;  // DMA instructions per wave per stage
+  constexpr int kStage = TA::kBytes + TB::kBytes;
+  __shared__ __attribute__((aligned(256))) char lds[2 * kStage];
 
   int tm, tn;
   tile_coords<BM, BN>(a, tm, tn);
@@ -430,50 +519,10 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_dma(GemmArgs a) {
   }
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  // The wave index as a uniform (SGPR) value: the DMA's LDS address (M0) is then
-  // computed on the scalar unit, not read back from a vector register per copy.
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int g = lane >> 5, r = lane & 31;
 
-  TA ta;
-  TB tb;
-  ta.init(A, a.lda, a.M, m0, wave_s, lane);
-  tb.init(B, a.ldb, a.N, n0, wave_s, lane);
-
-  // Per-lane fragment offsets (floats) inside a stage's A / B tile.
-  // K-contiguous: slab s reads unit 4 (r % 16) + ((2 s + g) ^ swz(r % 16)) of
-  // 16-row block (row / 16); MN-contiguous: k-row 8 s + 4 g + j, float
-  // ((mbase / 4) ^ 8 g) * 4 + r.
-  int offA[2], offB[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const int u = 4 * (4 * (r & 15) + ((2 * s + g) ^ swz(r & 15))) + (r >> 4) * 256;
-    offA[s] = u + wm * (BM / 2) * 16;
-    offB[s] = u + wn * (BN / 2) * 16;
-  }
-  const int mbA = (wm * (BM / 2)) >> 2, mbB = (wn * (BN / 2)) >> 2;
-  // A fragments of slab s.  With kPermA, MFMA tile i's row slot x holds tile
-  // row wm * (BM / 2) + 4x + i (not 32i + x): the b128 at k-row 8s + 4g + j,
-  // chunk mbA + r (swizzled as stored) is then lane (g, r)'s k-step-j value
-  // for all four tiles.  Each output element sums the same products in the
-  // same k order either way; only the rows' places in the registers move,
-  // which the epilogue undoes.
-  auto load_a = [&](const float* st, int s, f32x4 (&fa)[FI]) {
-    if constexpr (kPermA) {
-      const int off = 4 * ((mbA + r) ^ (8 * g));
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(st + (8 * s + 4 * g + j) * BM + off);
-#pragma unroll
-        for (int i = 0; i < FI; ++i) fa[i][j] = v[i];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < FI; ++i) fa[i] = dma_frag<A_KC, BM>(st, offA[s], i, s, g, r, mbA);
-    }
-  };
   f32x16 acc[FI][FJ];
 #pragma unroll
   for (int i = 0; i < FI; ++i)
@@ -482,179 +531,225 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_dma(GemmArgs a) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  const int64_t nk = K / 16;
+  const int64_t nk = (K + 15) / 16;
+  const int ra = g * TA::kHalf + (wm * (BM / 2) + r) * 16;
+  const int rb = TA::kBytes + g * TB::kHalf + (wn * (BN / 2) + r) * 16;
+  const unsigned start = (__builtin_popcountll(bz) & 1) ? 0x80000000u : 0u;
   if (nk > 0) {
-    ta.issue(lds, 0, wave_s);
-    tb.issue(lds + TA::kFloats, 0, wave_s);
-  }
-  if (nk > 1) {
-    ta.issue(lds + kStage, 1, wave_s);
-    tb.issue(lds + kStage + TA::kFloats, 1, wave_s);
-    wait_vm_lgkm0<NI>();
-  } else {
-    wait_vm_lgkm0<0>();
-  }
-  block_barrier();
-  float* st0 = lds;
-  f32x4 fa0[FI], fb0[FJ], fa1[FI], fb1[FJ];
-  load_a(st0, 0, fa0);
-#pragma unroll
-  for (int j = 0; j < FJ; ++j) fb0[j] = dma_frag<B_KC, BN>(st0 + TA::kFloats, offB[0], j, 0, g, r, mbB);
-
-  // The k loop is peeled: stages 0 .. nk-3 issue the DMA of the stage two
-  // ahead, the last two none, so the DMA instructions sit in straight-line
-  // code the scheduler can spread among the MFMAs (one burst of them holds up
-  // this wave's MFMA issue while the memory pipe takes them).  Where: among
-  // the slab-1 MFMAs before the barrier (the late form), or among the slab-0
-  // MFMAs.  With buffer-resource copies the late form is 0.2-1.7% faster on
-  // both tile shapes; with 64-bit-address copies the slab-0 form was 1-3%
-  // faster on 128-row tiles.  The arithmetic is the same either way.
-  constexpr bool kLateDma = BUF || BM == 256;
-  int ic = 0;  // kt % 3
-  auto stage = [&](int64_t kt, auto with_dma) {
-    constexpr bool kDma = decltype(with_dma)::value;
-    float* cur = lds + ic * kStage;
-    float* nxt = lds + (ic == 2 ? 0 : ic + 1) * kStage;
-    float* nx2 = lds + (ic == 0 ? 2 : ic - 1) * kStage;
-    load_a(cur, 1, fa1);
-#pragma unroll
-    for (int j = 0; j < FJ; ++j) fb1[j] = dma_frag<B_KC, BN>(cur + TA::kFloats, offB[1], j, 1, g, r, mbB);
-    if constexpr (kDma && !kLateDma) {
-      ta.issue(nx2, kt + 2, wave_s);
-      tb.issue(nx2 + TA::kFloats, kt + 2, wave_s);
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int i = 0; i < FI; ++i)
-#pragma unroll
-        for (int j = 0; j < FJ; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa0[i][s], fb0[j][s], acc[i][j], 0, 0, 0);
-    if constexpr (kDma && !kLateDma)
-      interleave2<NR, NI, NM>();
-    else
-      interleave_mfma_first<NR, NM, 0x100>();
-    if constexpr (kDma && kLateDma) {
-      ta.issue(nx2, kt + 2, wave_s);
-      tb.issue(nx2 + TA::kFloats, kt + 2, wave_s);
-    }
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int i = 0; i < FI; ++i)
-#pragma unroll
-        for (int j = 0; j < FJ; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa1[i][s], fb1[j][s], acc[i][j], 0, 0, 0);
-    if constexpr (kDma && kLateDma) interleave<NI, NM / 2, 0x020>();
-    // Stage kt+1's DMA has landed (only stage kt+2's may still be in flight)
-    // and every wave is done reading stage kt's buffer.
-    if constexpr (kDma)
-      wait_vm_lgkm0<NI>();
-    else
-      wait_vm_lgkm0<0>();
+    const int64_t pairs = (nk + 1) / 2;  // an odd nk's last stage is all zeros
+    const int64_t turn[3] = {(pairs * 212) >> 10, (pairs * 724) >> 10, pairs};
+    unsigned sign;  // of the values stored, which belong to pair `at`
+    const auto sign_at = [&](int64_t at) {
+      sign = start ^ (at >= turn[0] && at < turn[1] ? 0x80000000u : 0u);
+    };
+    sign_at(0);
+    TA ta;
+    TB tb;
+    ta.init(A, a.lda, a.M, K, m0, wave, lane);
+    tb.init(B, a.ldb, a.N, K, n0, wave, lane);
+    int64_t klane = K - 4 * (lane & 3);  // TAIL: k left from this lane's quad on
+    ta.load_all();
+    tb.load_all();
+    ta.template store_all<false, TAIL>(lds, klane > 0, sign);
+    tb.template store_all<true, TAIL>(lds + TA::kBytes, klane > 0, sign);
+    ta.load_all();
+    tb.load_all();
+    wait_lgkm0();
     block_barrier();
-    load_a(nxt, 0, fa0);
+    bf16x8 fa[2][3], fb[2][FJ][3];
 #pragma unroll
-    for (int j = 0; j < FJ; ++j) fb0[j] = dma_frag<B_KC, BN>(nxt + TA::kFloats, offB[0], j, 0, g, r, mbB);
+    for (int p = 0; p < 3; ++p) fa[0][p] = TA::frag(lds, ra, p, 0);
 #pragma unroll
-    for (int s = 2; s < 4; ++s)
+    for (int j = 0; j < FJ; ++j)
 #pragma unroll
-      for (int i = 0; i < FI; ++i)
-#pragma unroll
-        for (int j = 0; j < FJ; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa1[i][s], fb1[j][s], acc[i][j], 0, 0, 0);
-    interleave<NR, NM / 2, 0x100>();
-    ic = ic == 2 ? 0 : ic + 1;
-  };
-  int64_t kt = 0;
-  for (; kt + 2 < nk; ++kt) stage(kt, std::true_type{});
-  for (; kt < nk; ++kt) stage(kt, std::false_type{});
+      for (int p = 0; p < 3; ++p) fb[0][j][p] = TB::frag(lds, rb, p, j);
 
-  if constexpr (BUF) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    // Stores (and the beta term's loads) through buffer resources based at
-    // this wave's first output row of C (and of D): a row's byte offset splits
-    // into a uniform part (the MFMA register's row slot, in an SGPR) and the
-    // lane's part (computed once), with no 64-bit address arithmetic per
-    // element.  Rows at or past M are skipped by an explicit test, made only on
-    // the wave tiles that reach M.  Same values as the form below.
-    const int wm_s = wave_s >> 1, wn_s = wave_s & 1;
-    const int64_t rw0 = m0 + wm_s * (BM / 2), cw0 = n0 + wn_s * (BN / 2);
-    if (rw0 < a.M) {
-      const float* Dm = a.D ? a.D : C;
-      const int64_t ldd = a.D ? a.ldd : a.ldc;
-      const __amdgpu_buffer_rsrc_t rc =
-          __builtin_amdgcn_make_buffer_rsrc(C + rw0 * a.ldc + cw0, 0, 0x7fffffff, 0x00020000);
-      const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<float*>(Dm + rw0 * ldd + cw0), 0, 0x7fffffff, 0x00020000);
-      const int lrow = kPermA ? 16 * g : 4 * g;  // the lane's part of the row
-      const int lc = static_cast<int>((lrow * a.ldc + r) * 4);
-      const int ld = static_cast<int>((lrow * ldd + r) * 4);
-      const int rows_left = static_cast<int>(min(a.M - rw0, int64_t{BM}));
-      // CHECKED: the wave tile reaches M.  BETA: the beta term is read, all 16
-      // values of an MFMA tile before the first is used (one wait per tile).
-      auto store_all = [&](auto checked, auto with_beta) {
-        constexpr bool kChecked = decltype(checked)::value, kBeta = decltype(with_beta)::value;
+    // One stage: FI groups of 6 FJ MFMAs, one group per 32-row tile of A.
+    // Between them, in this order: the split and store of the next stage's
+    // fetched values, each followed by the fetch of the stage after it; a
+    // barrier before the last group; the next stage's first fragments.
+    auto stage = [&](auto odd) {
+      constexpr int kOdd = decltype(odd)::value;
+      constexpr int kGroup = 6 * FJ;
+      constexpr int kSlots = (FI - 1) * kGroup - (FI > 2 ? 8 : 2);  // for the splits
+      constexpr int kQuads = TA::P + TB::P;
+      constexpr int kWork = kQuads * TA::kSteps;
+      const char* cur = lds + kOdd * kStage;
+      char* nxt = lds + (1 - kOdd) * kStage;
+      if (TAIL) klane -= 16;
+      SplitWork w;
 #pragma unroll
-        for (int j = 0; j < FJ; ++j) {
-          if (cw0 + j * 32 + r >= a.N) continue;
+      for (int i = 0; i < FI; ++i) {
+        constexpr int pa[6] = {0, 1, 2, 0, 1, 0}, pb[6] = {2, 1, 0, 1, 0, 0};  // smallest first
 #pragma unroll
-          for (int i = 0; i < FI; ++i) {
-            float d[16];
+        for (int t = 0; t < 6; ++t)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-              const int ru = kPermA ? 4 * (8 * (e >> 2) + (e & 3)) + i
-                                    : i * 32 + 8 * (e >> 2) + (e & 3);
-              d[e] = 0.f;
-              if (kBeta && !(kChecked && ru + lrow >= rows_left))
-                d[e] = __builtin_bit_cast(
-                    float, __builtin_amdgcn_raw_buffer_load_b32(
-                               rd, ld + 128 * j, static_cast<int>(ru * ldd * 4), 0));
+          for (int j = 0; j < FJ; ++j) {
+            const int in = t * FJ + j, m = i * kGroup + in;
+            if (i == FI - 1 && in == 0) {
+              wait_lgkm0();
+              block_barrier();
             }
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-              // the row slot's uniform part; the lane's part is in lc / ld
-              const int ru = kPermA ? 4 * (8 * (e >> 2) + (e & 3)) + i
-                                    : i * 32 + 8 * (e >> 2) + (e & 3);
-              if (kChecked && ru + lrow >= rows_left) continue;
-              const float v = a.alpha * acc[i][j][e];
-              const float out = kBeta ? v + a.beta * d[e] : v;
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, out), rc,
-                                                    lc + 128 * j,
-                                                    static_cast<int>(ru * a.ldc * 4), 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                fa[i & 1][pa[t]], fb[kOdd][j][pb[t]], acc[i][j], 0, 0, 0);
+            if (i < FI - 1) {
+              if (in < 3) fa[(i + 1) & 1][in] = TA::frag(cur, ra, in, i + 1);
+            } else if (in < 3 + 3 * FJ) {
+              if (in < 3) fa[0][in] = TA::frag(nxt, ra, in, 0);
+              else fb[1 - kOdd][(in - 3) / 3][(in - 3) % 3] = TB::frag(nxt, rb, (in - 3) % 3, (in - 3) / 3);
             }
+            if (m < kSlots) {
+#pragma unroll
+              for (int s = m * kWork / kSlots; s < (m + 1) * kWork / kSlots; ++s) {
+                const int q = s / TA::kSteps, st = s % TA::kSteps;
+                if (q < TA::P)
+                  ta.template split_step<false, TAIL>(w, q, st, nxt, klane > 0, sign);
+                else
+                  tb.template split_step<true, TAIL>(w, q - TA::P, st, nxt + TA::kBytes,
+                                                     klane > 0, sign);
+                if (s == TA::P * TA::kSteps - 1) ta.load_all();
+                if (s == kWork - 1) tb.load_all();
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
           }
-        }
-      };
-      const bool full = rows_left >= BM / 2;
-      if (a.beta != 0.f) {
-        if (full) store_all(std::false_type{}, std::true_type{});
-        else store_all(std::true_type{}, std::true_type{});
-      } else {
-        if (full) store_all(std::false_type{}, std::false_type{});
-        else store_all(std::true_type{}, std::false_type{});
+      }
+    };
+    int64_t p = 0;
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+      while (p < turn[part]) {
+        stage(std::integral_constant<int, 0>{});
+        sign_at(++p);
+        stage(std::integral_constant<int, 1>{});
+      }
+      if (part < 2) {
+#pragma unroll
+        for (int i = 0; i < FI; ++i)
+#pragma unroll
+          for (int j = 0; j < FJ; ++j) acc[i][j] = -acc[i][j];
       }
     }
-#endif
-  } else {
+  }
+
+  // The lane's place in the output: register e of tile (i, j) is row slot
+  // x = 8 (e / 4) + 4 g + e % 4 of MFMA tile i and column slot r of tile j.
+  const int64_t rw0 = m0 + wm * (BM / 2), cw0 = n0 + wn * (BN / 2);
+  if (rw0 >= a.M || cw0 >= a.N) return;
+  const auto row_of = [&](int i, int e) {  // its uniform part; the lane's is lrow
+    const int x = 8 * (e >> 2) + (e & 3);
+    return A_KC ? i * 32 + x : FI * x + i;
+  };
+  const auto col_of = [&](int j) { return B_KC ? j * 32 + r : FJ * r + j; };
+  const int lrow = A_KC ? 4 * g : FI * 4 * g;
+  const int rows_left = static_cast<int>(min(a.M - rw0, int64_t{BM}));
+  const int cols_left = static_cast<int>(min(a.N - cw0, int64_t{BN}));
+
+  // (Values are taken out before their bits: a bit_cast of a vector element
+  // reads element 0.)
+  unsigned most = 0;
+#pragma unroll
+  for (int i = 0; i < FI; ++i)
+#pragma unroll
+    for (int j = 0; j < FJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float f = acc[i][j][e];
+        most = max(most, out_of_range(__builtin_bit_cast(unsigned, f)));
+      }
+  bool redo = false;
+  if (__any(most >= kOutOfRange)) {
 #pragma unroll
     for (int i = 0; i < FI; ++i)
 #pragma unroll
-      for (int j = 0; j < FJ; ++j) {
-        const int64_t col = n0 + wn * (BN / 2) + j * 32 + r;
-        if (col >= a.N) continue;
+      for (int j = 0; j < FJ; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const int x = 8 * (e >> 2) + 4 * g + (e & 3);  // the MFMA tile's row slot
-          const int64_t row = m0 + wm * (BM / 2) + (kPermA ? 4 * x + i : i * 32 + x);
-          if (row < a.M) {
-            float* dst = C + row * a.ldc + col;
-            const float v = a.alpha * acc[i][j][e];
-            *dst = (a.beta != 0.f) ? v + a.beta * *addend(a, dst, row, col) : v;
-          }
+          const float f = acc[i][j][e];
+          redo |= f != 0.f && out_of_range(__builtin_bit_cast(unsigned, f)) >= kOutOfRange;
+        }
+  }
+  if (__builtin_expect(__any(redo), 0)) {
+    // This wave's tile in fp32 from global memory, 32x32 at a time.
+    for (int t = 0; t < FI * FJ; ++t) {
+      const int i = t / FJ, j = t % FJ;
+      const int64_t ar = min(rw0 + (A_KC ? i * 32 + r : FI * r + i), a.M - 1);
+      const int64_t bc = min(cw0 + col_of(j), a.N - 1);
+      const float* pa = A_KC ? A + ar * a.lda : A + ar;
+      const float* pb = B_KC ? B + bc * a.ldb : B + bc;
+      const int64_t sa = A_KC ? 1 : a.lda, sb = B_KC ? 1 : a.ldb;
+      f32x16 v;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v[e] = 0.f;
+      for (int64_t k = g; k < K + g; k += 2) {
+        const float x = k < K ? pa[k * sa] : 0.f, y = k < K ? pb[k * sb] : 0.f;
+        v = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, v, 0, 0, 0);
+      }
+      if (col_of(j) >= cols_left) continue;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int64_t row = rw0 + row_of(i, e) + lrow, col = cw0 + col_of(j);
+        if (row >= a.M) continue;
+        float* dst = C + row * a.ldc + col;
+        const float x = a.alpha * v[e];
+        *dst = (a.beta != 0.f) ? x + a.beta * *addend(a, dst, row, col) : x;
+      }
+    }
+    return;
+  }
+
+  const float back = start ? -1.f : 1.f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  // Stores (and the beta term's loads) through buffer resources based at this
+  // wave's first output row of C (and of D): a row's byte offset splits into a
+  // uniform part (in an SGPR) and the lane's part (computed once).
+  const float* Dm = a.D ? a.D : C;
+  const int64_t ldd = a.D ? a.ldd : a.ldc;
+  const __amdgpu_buffer_rsrc_t rc =
+      __builtin_amdgcn_make_buffer_rsrc(C + rw0 * a.ldc + cw0, 0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(Dm + rw0 * ldd + cw0), 0, 0x7fffffff, 0x00020000);
+  const int lc = static_cast<int>(lrow * a.ldc * 4), ld = static_cast<int>(lrow * ldd * 4);
+  // CHECKED: the wave tile reaches M.  BETA: the beta term is read, all 16
+  // values of an MFMA tile before the first is used (one wait per tile).
+  auto store_all = [&](auto checked, auto with_beta) {
+    constexpr bool kChecked = decltype(checked)::value, kBeta = decltype(with_beta)::value;
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) {
+      const int col = col_of(j);
+      if (col >= cols_left) continue;
+#pragma unroll
+      for (int i = 0; i < FI; ++i) {
+        float d[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int ru = row_of(i, e);
+          d[e] = 0.f;
+          if (kBeta && !(kChecked && ru + lrow >= rows_left))
+            d[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                 rd, ld + 4 * col, static_cast<int>(ru * ldd * 4), 0));
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int ru = row_of(i, e);
+          if (kChecked && ru + lrow >= rows_left) continue;
+          const float v = a.alpha * __builtin_fmaf(back, acc[i][j][e], 0.f);  // +0 for a zero
+          const float out = kBeta ? v + a.beta * d[e] : v;
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, out), rc, lc + 4 * col,
+                                                static_cast<int>(ru * a.ldc * 4), 0);
         }
       }
+    }
+  };
+  const bool full = rows_left >= BM / 2;
+  if (a.beta != 0.f) {
+    if (full) store_all(std::false_type{}, std::true_type{});
+    else store_all(std::true_type{}, std::true_type{});
+  } else {
+    if (full) store_all(std::false_type{}, std::false_type{});
+    else store_all(std::true_type{}, std::false_type{});
   }
+#endif
 }
 
 // C = alpha * sum_{s<S} P[s] + beta * D (D = C when null), the split partials
@@ -798,17 +893,23 @@ int launch_skinny(const float* A, int64_t lda, const float* B, int64_t ldb, floa
   return launch_status();
 }
 
-// Launch plan for one call.
+int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The K splits a product can have, which size its workspace, and the plan of
+// gemm_f32_mfma.
 struct Plan {
-  bool big;         // 256x128 tiles (else 128x128)
+  bool big;         // unsplit: 256x128 tiles (else 128x128)
   int64_t splits;   // 1 = no K split
   int64_t kchunk;   // k per split (multiple of kBK)
 };
 
-int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
 Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
   Plan p{false, 1, 0};
+  const auto split = [&](int64_t s) {
+    p.kchunk = cdiv(cdiv(K, s), kBK) * kBK;
+    p.splits = cdiv(K, p.kchunk);
+    return p;
+  };
   const int64_t big_tiles = cdiv(M, 256) * cdiv(N, 128) * batch;
   if (big_tiles >= 4 * kCUs) {  // at least two full waves of 2 blocks per CU
     p.big = true;
@@ -816,35 +917,92 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
   }
   const int64_t tiles = cdiv(M, 128) * cdiv(N, 128) * batch;
   const int64_t target = 6 * kCUs;  // two waves of 3 blocks per CU
-  // K chunks of at least 1024 from K = 4096 up.  A grid that would fill at
-  // most half the CUs (e.g. the projections of a short prefill, M = 128) is
-  // latency-bound on its one pass over K: chunks of at least 256 from K = 512.
+  // K chunks of at least 1024 from K = 2560 up (5000x960x2560 unsplit takes
+  // 170 us, in three chunks 152; 4096x1024x3072 151 and 147 in two).  A grid
+  // that would fill at most half the CUs (e.g. the projections of a short
+  // prefill, M = 128) is latency-bound on its one pass over K: from K = 512,
+  // up to eight chunks of at least 96, then chunks of 256 (256x576x576 in six
+  // chunks 12.7 us, in two 18.4; 128x1024x1024 in eight 14.6, in four 18.3).
   const bool few = 2 * tiles <= kCUs;
-  const int64_t min_chunk = few ? 256 : 1024;
-  // A K split on 256x128 tiles, in chunks of at least 1024, when a whole
-  // number of waves of them (two per CU) is at least two waves: 2-4% faster
-  // than the 128x128 split on the weight-gradient shapes that allows (e.g.
-  // 1024x2048, 2048x2048 and 6144x2048 over 32768 tokens), which a partial
-  // last wave made up to 8% slower.
+  // From K = 4096, chunks of at least 1024 in a whole number of waves of
+  // 256x128 tiles (two per CU), at least two.
   if (batch == 1 && K >= 4096) {
     int64_t s = cdiv(4 * kCUs, big_tiles);
     while (s < 16 && (big_tiles * s) % (2 * kCUs) != 0) ++s;
-    if (s >= 2 && s <= K / 1024 && (big_tiles * s) % (2 * kCUs) == 0) {
-      p.big = true;
-      p.kchunk = cdiv(cdiv(K, s), kBK) * kBK;
-      p.splits = cdiv(K, p.kchunk);
-      return p;
-    }
+    if (s >= 2 && s <= K / 1024 && (big_tiles * s) % (2 * kCUs) == 0) return split(s);
   }
-  if (batch == 1 && tiles < target && K >= (few ? 2 * min_chunk : 4096)) {
-    int64_t s = std::min<int64_t>(16, cdiv(target, tiles));
-    s = std::min<int64_t>(s, K / min_chunk);
-    if (s >= 2) {
-      p.kchunk = cdiv(cdiv(K, s), kBK) * kBK;
-      p.splits = cdiv(K, p.kchunk);
-    }
+  if (batch == 1 && tiles < target && K >= (few ? 512 : 2560)) {
+    const int64_t chunk = few ? std::min<int64_t>(256, std::max<int64_t>(96, K / 8)) : 1024;
+    const int64_t s = std::min({int64_t{16}, cdiv(target, tiles), K / chunk});
+    if (s >= 2) return split(s);
   }
   return p;
+}
+
+// Launch plan for gemm_f32_split: the tile shape and the K split of least
+// predicted time.  The prediction counts what the busiest CU does, in
+// microseconds: whole rounds of as many blocks as fit a CU, then what is
+// left, a stage of 16 k costing `stage[n - 1]` while n blocks share the CU
+// (`alone` when at most half the CUs have one, and clocks are high), and a
+// round `ends` more for its first loads and its stores, which only other
+// blocks on the same CU can cover.  A split adds its reduction: one launch
+// and S + 1 planes of C through HBM.  The constants are fitted to times of
+// 59 products (M, N 32 to 151936, K 64 to 151936, all three layouts) on every
+// tile with 1 to 16 splits; choosing by them is on average 0.5% slower than
+// the best of those, at worst 6%.
+struct SplitPlan {
+  int tile;         // index into kTiles
+  int64_t splits;   // 1 = no K split
+  int64_t kchunk;   // k per split, whole pairs of stages
+};
+struct TileCost {
+  int64_t bm, bn;
+  int per_cu;
+  double stage[3], alone, ends;
+};
+constexpr TileCost kTiles[3] = {{128, 128, 3, {0.67, 1.12, 1.89}, 0.53, 3.71},
+                                {256, 128, 2, {1.11, 2.19}, 0.78, 7.0},
+                                {256, 256, 1, {1.92}, 1.38, 27.3}};
+
+double predicted_us(const TileCost& t, int64_t M, int64_t N, int64_t K, int64_t batch,
+                    int64_t splits) {
+  const double stages = static_cast<double>(cdiv(K, 16));
+  const int64_t blocks = cdiv(M, t.bm) * cdiv(N, t.bn) * batch * splits;
+  const int64_t round = int64_t{t.per_cu} * kCUs;
+  double us = static_cast<double>(blocks / round) * (t.stage[t.per_cu - 1] * stages + t.ends);
+  const int64_t rest = blocks % round;
+  if (rest > 0) {
+    const int64_t n = cdiv(rest, kCUs);
+    if (blocks == rest && 2 * rest <= kCUs)
+      us += t.alone * stages + 3.0;
+    else
+      us += t.stage[n - 1] * stages + t.ends * static_cast<double>(n) / t.per_cu;
+  }
+  return us;
+}
+
+// `room`: the partial products that the workspace holds; `tiles`: the first
+// of kTiles that may be used.
+// From K = 4096 the split is all of `room`: shorter partial sums are also what
+// keeps the error of long ones down (a weight gradient's terms vary along the
+// tokens; 1024x2048x32768 in 8 chunks instead of 16 was 1.5 times further
+// from 64-bit sums, and 4% faster).
+SplitPlan make_split_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t room,
+                          int tiles) {
+  SplitPlan best{0, 1, 0};
+  double least = 1e30;
+  for (int t = 0; t < tiles; ++t)
+    for (int64_t s = K >= 4096 ? room : 1; s <= room; ++s) {
+      const int64_t chunk = s > 1 ? cdiv(cdiv(K, s), 32) * 32 : K;
+      const int64_t n = s > 1 ? cdiv(K, chunk) : 1;  // at most s
+      double us = predicted_us(kTiles[t], M, N, chunk, batch, n);
+      if (n > 1) us += 2.45 + static_cast<double>((n + 1) * M * N) * 4 / 5.68e6;
+      if (us < least) {
+        least = us;
+        best = SplitPlan{t, n, n > 1 ? chunk : 0};
+      }
+    }
+  return best;
 }
 
 template <bool A_KC, bool B_KC, int BM, int BN, int OCC>
@@ -868,28 +1026,48 @@ int launch_t(GemmArgs a, bool a_kc, bool b_kc, int64_t ny, bool vec, hipStream_t
 }
 
 template <bool A_KC, bool B_KC, int BM, int BN, int OCC>
-int launch_dma_t(GemmArgs a, int64_t ny, hipStream_t st) {
+int launch_split_t(GemmArgs a, int64_t ny, hipStream_t st) {
   a.tiles_m = static_cast<int>(cdiv(a.M, BM));
   a.tiles_n = static_cast<int>(cdiv(a.N, BN));
   dim3 grid(static_cast<unsigned>(a.tiles_m) * a.tiles_n, static_cast<unsigned>(ny));
-  // Largest byte offset a block's buffer resource must reach: BM (BN) rows of
-  // K plus K, or K rows of lda (ldb) plus the tile's columns.
-  const int64_t span_a = A_KC ? BM * a.lda + a.K : a.K * a.lda + BM;
-  const int64_t span_b = B_KC ? BN * a.ldb + a.K : a.K * a.ldb + BN;
-  const int64_t span_c = BM * std::max(a.ldc, a.D ? a.ldd : int64_t{0});  // the epilogue's rows
-  if (4 * std::max({span_a, span_b, span_c}) < (int64_t{1} << 31) - 256)
-    gemm_f32_dma<A_KC, B_KC, BM, BN, OCC, true><<<grid, kThreads, 0, st>>>(a);
+  // Stages run in pairs: a K-contiguous operand has to be masked past K unless
+  // every split is whole pairs (an MN-contiguous one ends where memory says).
+  const bool whole = (a.kchunk > 0 ? a.kchunk : a.K) % 32 == 0 && a.K % 32 == 0 &&
+                     !(a.dyn && a.dyn_dim == 1);
+  if ((A_KC || B_KC) && !whole)
+    gemm_f32_split<A_KC, B_KC, BM, BN, OCC, true><<<grid, kThreads, 0, st>>>(a);
   else
-    gemm_f32_dma<A_KC, B_KC, BM, BN, OCC, false><<<grid, kThreads, 0, st>>>(a);
+    gemm_f32_split<A_KC, B_KC, BM, BN, OCC, false><<<grid, kThreads, 0, st>>>(a);
   return launch_status();
 }
 
 template <int BM, int BN, int OCC>
-int launch_dma(const GemmArgs& a, bool a_kc, bool b_kc, int64_t ny, hipStream_t st) {
-  if (a_kc && b_kc) return launch_dma_t<true, true, BM, BN, OCC>(a, ny, st);
-  if (a_kc && !b_kc) return launch_dma_t<true, false, BM, BN, OCC>(a, ny, st);
-  if (!a_kc && !b_kc) return launch_dma_t<false, false, BM, BN, OCC>(a, ny, st);
-  return launch_dma_t<false, true, BM, BN, OCC>(a, ny, st);
+int launch_split_tile(const GemmArgs& a, bool a_kc, bool b_kc, int64_t ny, hipStream_t st) {
+  if (a_kc && b_kc) return launch_split_t<true, true, BM, BN, OCC>(a, ny, st);
+  if (a_kc && !b_kc) return launch_split_t<true, false, BM, BN, OCC>(a, ny, st);
+  if (!a_kc && !b_kc) return launch_split_t<false, false, BM, BN, OCC>(a, ny, st);
+  return launch_split_t<false, true, BM, BN, OCC>(a, ny, st);
+}
+
+int launch_split(const GemmArgs& a, int tile, bool a_kc, bool b_kc, int64_t ny, hipStream_t st) {
+  return tile == 0   ? launch_split_tile<128, 128, 3>(a, a_kc, b_kc, ny, st)
+         : tile == 1 ? launch_split_tile<256, 128, 2>(a, a_kc, b_kc, ny, st)
+                     : launch_split_tile<256, 256, 1>(a, a_kc, b_kc, ny, st);
+}
+
+// How many of kTiles gemm_f32_split can use for these operands: none unless
+// their rows are float4 rows that end on a whole float4; else those for which
+// every byte offset inside a block's operand stage and output tile (the
+// tile's rows of a K-contiguous operand and of C, 16 k of the other) stays
+// below 2^31.
+int split_tiles(const GemmArgs& a, bool a_kc, bool b_kc, bool vec) {
+  if (!vec || (a_kc ? a.K : a.M) % 4 != 0 || (b_kc ? a.K : a.N) % 4 != 0) return 0;
+  const auto fits = [&](int64_t rows) {
+    const int64_t top = (int64_t{1} << 29) - 1024;  // floats
+    return (a_kc ? rows - 1 : 16) * a.lda < top && (b_kc ? rows - 1 : 16) * a.ldb < top &&
+           rows * std::max(a.ldc, a.D ? a.ldd : int64_t{0}) < top;
+  };
+  return fits(256) ? 3 : fits(128) ? 1 : 0;
 }
 
 int check_args(int transa, int transb, int64_t M, int64_t N, int64_t K, const float* A,
@@ -938,27 +1116,30 @@ int gemm_run(int transa, int transb, int64_t M, int64_t N, int64_t K, float alph
                            : launch_skinny<8>;
     return skinny(A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, D, ldd, st);
   }
-  Plan p = make_plan(M, N, K, batch);
-  if (p.splits > 1 &&
-      ((dyn && dyn_dim == 1) || !workspace ||
-       workspace_bytes < static_cast<size_t>(p.splits * M * N) * sizeof(float)))
-    p.splits = 1;  // no room for partials, or K itself is decided on the device
-  if (p.splits > 1) {
+  // Partial products need room for themselves, and a K known on the host.
+  const Plan p = make_plan(M, N, K, batch);
+  const bool room = p.splits > 1 && !(dyn && dyn_dim == 1) && workspace &&
+                    workspace_bytes >= static_cast<size_t>(p.splits * M * N) * sizeof(float);
+  const int tiles = split_tiles(a, a_kc, b_kc, vec);
+  const bool fast = tiles > 0;
+  SplitPlan sp{0, 1, 0};
+  if (fast) sp = make_split_plan(M, N, K, batch, room ? p.splits : 1, tiles);
+  const int64_t splits = fast ? sp.splits : room ? p.splits : 1;
+  const int64_t kchunk = fast ? sp.kchunk : p.kchunk;
+  if (splits > 1) {
     // Split s computes A[:, s*kchunk ...] B[s*kchunk ..., :] into plane s.
-    GemmArgs sp = a;
-    sp.C = static_cast<float*>(workspace);
-    sp.ldc = N;
-    sp.sA = a_kc ? p.kchunk : p.kchunk * lda;
-    sp.sB = b_kc ? p.kchunk : p.kchunk * ldb;
-    sp.sC = M * N;
-    sp.kchunk = p.kchunk;
-    sp.alpha = 1.f;
-    sp.beta = 0.f;
-    const bool dma = vec && p.kchunk % 16 == 0 && K % 16 == 0 && (a_kc || M % 4 == 0) &&
-                     (b_kc || N % 4 == 0);
-    if ((rc = dma ? (p.big ? launch_dma<256, 128, 2>(sp, a_kc, b_kc, p.splits, st)
-                           : launch_dma<128, 128, 3>(sp, a_kc, b_kc, p.splits, st))
-                  : launch_t<128, 128, 3>(sp, a_kc, b_kc, p.splits, vec, st)))
+    GemmArgs pa = a;
+    pa.C = static_cast<float*>(workspace);
+    pa.ldc = N;
+    pa.sA = a_kc ? kchunk : kchunk * lda;
+    pa.sB = b_kc ? kchunk : kchunk * ldb;
+    pa.sC = M * N;
+    pa.kchunk = kchunk;
+    pa.alpha = 1.f;
+    pa.beta = 0.f;
+    pa.D = nullptr;
+    if ((rc = fast ? launch_split(pa, sp.tile, a_kc, b_kc, splits, st)
+                   : launch_t<128, 128, 3>(pa, a_kc, b_kc, splits, vec, st)))
       return rc;
     const bool rvec = (N % 4 == 0) && (ldc % 4 == 0) && aligned16(C) &&
                       (!D || (ldd % 4 == 0 && aligned16(D)));
@@ -967,19 +1148,15 @@ int gemm_run(int transa, int transb, int64_t M, int64_t N, int64_t K, float alph
     const int64_t* rdyn = dyn_dim == 0 ? dyn : nullptr;
     if (rvec)
       splitk_reduce<true><<<blocks, kThreads, 0, st>>>(static_cast<const float*>(workspace), C, M,
-                                                       N, ldc, static_cast<int>(p.splits),
-                                                       alpha, beta, rdyn, dyn_base, D, ldd);
+                                                       N, ldc, static_cast<int>(splits), alpha,
+                                                       beta, rdyn, dyn_base, D, ldd);
     else
       splitk_reduce<false><<<blocks, kThreads, 0, st>>>(static_cast<const float*>(workspace), C,
-                                                        M, N, ldc, static_cast<int>(p.splits),
-                                                        alpha, beta, rdyn, dyn_base, D, ldd);
+                                                        M, N, ldc, static_cast<int>(splits), alpha,
+                                                        beta, rdyn, dyn_base, D, ldd);
     return launch_status();
   }
-  const bool dma = vec && K % 16 == 0 && (a_kc || M % 4 == 0) && (b_kc || N % 4 == 0) &&
-                   (batch == 1 || (sA % 4 == 0 && sB % 4 == 0));
-  if (dma && p.big) return launch_dma<256, 128, 2>(a, a_kc, b_kc, batch, st);
-  if (dma) return launch_dma<128, 128, 3>(a, a_kc, b_kc, batch, st);
-  if (dyn) return EMBER_EINVAL;  // only the LDS-DMA kernels read a device-side extent
+  if (fast) return launch_split(a, sp.tile, a_kc, b_kc, batch, st);
   if (p.big) return launch_t<256, 128, 2>(a, a_kc, b_kc, batch, vec, st);
   return launch_t<128, 128, 3>(a, a_kc, b_kc, batch, vec, st);
 }
@@ -1024,7 +1201,7 @@ extern "C" int ember_gemm_f32_dyn(int transa, int transb, int64_t M, int64_t N, 
   int rc = check_args(transa, transb, M, N, K, A, lda, B, ldb, C, ldc, 1);
   if (rc) return rc;
   if (!count || (dim != 0 && dim != 1) || base < 0) return EMBER_EINVAL;
-  // The LDS-DMA kernels' conditions: 16-byte rows and K in whole 16-k stages.
+  // 16-byte rows, and K in whole 16-k stages.
   const bool a_kc = !transa, b_kc = transb != 0;
   if (!aligned16(A) || !aligned16(B) || lda % 4 != 0 || ldb % 4 != 0 || K % 16 != 0 ||
       (!a_kc && M % 4 != 0) || (!b_kc && N % 4 != 0))

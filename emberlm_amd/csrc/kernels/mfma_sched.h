@@ -43,32 +43,16 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (0 << 8));
 }
+// s_waitcnt lgkmcnt(0): this wave's LDS accesses are done (vmcnt and expcnt free).
+__device__ __forceinline__ void wait_lgkm0() {
+  __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4) | (0 << 8));
+}
 // Workgroup barrier with no implied memory wait (the waits above are explicit);
 // the empty asm keeps the compiler from moving memory accesses across it.
 __device__ __forceinline__ void block_barrier() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-}
-
-// NR LDS reads (mask 0x100) and NV VMEM loads (0x020) spread evenly among
-// NM MFMAs of the current region.
-template <int NR, int NV, int NM>
-__device__ __forceinline__ void interleave2() {
-  constexpr int per = NM / (NR + NV) > 0 ? NM / (NR + NV) : 1;
-  constexpr int n = NR > NV ? NR : NV;
-#pragma unroll
-  for (int t = 0; t < n; ++t) {
-    if (t < NR) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, per, 0);
-    }
-    if (t < NV) {
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, per, 0);
-    }
-  }
-  if (NM > (NR + NV) * per) __builtin_amdgcn_sched_group_barrier(0x008, NM - (NR + NV) * per, 0);
 }
 
 }  // namespace ember

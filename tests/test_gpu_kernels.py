@@ -744,6 +744,119 @@ def test_gemm_global_address_dma_bitwise_equals_buffer_dma(ta, tb, big):
     torch.cuda.empty_cache()
 
 
+def _gemm_dev(A, B, ta, tb, M, N, K, ws=True, beta=0.0, c=None):
+    """ember_gemm_f32_ws of device tensors -> device C, with or without its workspace."""
+    Cm = c if c is not None else empty((M, N))
+    need = capi.lib().ember_gemm_f32_workspace_bytes(M, N, K, 1) if ws else 0
+    buf = torch.empty(max(need // 4, 1), device="cuda")
+    call("ember_gemm_f32_ws", int(ta), int(tb), M, N, K, 1.0, p(A), A.shape[1], 0, p(B),
+         B.shape[1], 0, beta, p(Cm), N, 0, 1, p(buf) if need else None, need, None)
+    return Cm
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [
+    (12, 16, 4), (128, 128, 16), (132, 260, 36),      # 128x128: one tile, edges, k past a stage
+    (4, 4, 100), (500, 124, 1000),                    # few tiles: K splits, odd last chunk
+    (4092, 2052, 260), (4096, 4096, 48),              # larger tiles, ragged and whole, odd stages
+    (8196, 2564, 224),
+])
+def test_gemm_split_tile_edges_vs_float64(ta, tb, M, N, K):
+    """The split-operand kernel at its tiles' edges.  Bound: each of the 6 K / 16 sums
+    and K splits rounds to 2^-24 of a partial sum that is at most sqrt(K) of the terms'
+    size, so 2^-24 sqrt(6 K / 16 + 16) of the result's, and the operands are exact."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn((K, M) if ta else (M, K), device="cuda", generator=g)
+    B = torch.randn((N, K) if tb else (K, N), device="cuda", generator=g)
+    ref = (A.t() if ta else A).double().contiguous() @ (B.t() if tb else B).double().contiguous()
+    for ws in (True, False):
+        got = _gemm_dev(A, B, ta, tb, M, N, K, ws)
+        rel = ((got.double() - ref).norm() / ref.norm()).item()
+        assert rel <= 2.0 ** -24 * (6 * K / 16 + 16) ** 0.5, (rel, ws)
+        assert (got.double() - ref).abs().max().item() <= 2e-6 * K ** 0.5 * max(
+            1.0, ref.abs().max().item() / K ** 0.5)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+def test_gemm_split_small_terms_and_exact_products(ta, tb):
+    """All 24 bits of both operands count (K = 4 with one nonzero term is exact), and
+    a sum of like-signed products gathers no bias over columns."""
+    M, N = 64, 512
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(M, 1, device="cuda", generator=g)
+    a = torch.cat([x, torch.zeros(M, 3, device="cuda")], 1)
+    b = torch.ones(N, 4, device="cuda") * 3.0
+    A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+    got = _gemm_dev(A, B, ta, tb, M, N, 4)
+    assert torch.equal(got, (3.0 * x).expand(M, N))
+    K = 4096
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g)
+    A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+    ref = a.double() @ b.double().t().contiguous()
+    d = _gemm_dev(A, B, ta, tb, M, N, K, ws=False).double() - ref
+    # an unflipped kernel's mean is about -2.7e-7 of the mean size; noise is 1e-6 / sqrt(M N)
+    assert abs(d.mean().item()) <= 5e-8 * ref.abs().mean().item()
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(140, 132, 52), (4096, 2048, 64)])
+def test_gemm_split_nonfinite_and_range(ta, tb, M, N, K):
+    """Infinities, NaN, values past bf16's largest, overflow and products near the
+    smallest numbers come out as fp32 arithmetic has them, in their own rows and
+    columns only; zeros stay zeros."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a = torch.randn(M, K, device="cuda", generator=g)
+    b = torch.ones(N, K, device="cuda")
+    b[:, 1::2] = 0.0
+    a[3, 2] = float("inf")
+    a[5, 0] = float("-inf")
+    a[7, 4] = float("nan")
+    a[9, 6] = float("inf")
+    a[9, 8] = float("-inf")
+    a[11] = 0.0
+    a[11, 0] = 3.4e38                       # rounds to infinity in bf16
+    a[13] = 0.0
+    a[13, 0] = a[13, 2] = 3e38              # overflows
+    a[15] *= 2.0 ** -120                    # the last part of the split has no exponent left
+    a[17] = 0.0
+    b[21] *= 2.0 ** -130
+    A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+    got = _gemm_dev(A, B, ta, tb, M, N, K)
+    ref = a.double() @ b.double().t().contiguous()
+    ref = torch.where(ref.abs() > 3.4028235e38, torch.copysign(torch.full_like(ref, float("inf")), ref),
+                      ref)
+    assert torch.isnan(got[7]).all() and torch.isnan(got[9]).all()
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(got[torch.isinf(ref)].double(), ref[torch.isinf(ref)])
+    assert (got[17] == 0).all() and not torch.signbit(got[17]).any()
+    size = a.double().abs().masked_fill(~torch.isfinite(a), 0) @ b.double().t().contiguous()
+    # fp32 sums of K terms, and the smallest subnormal per term
+    assert ((got.double() - ref).abs()[fin] <= (K * 2.0 ** -24 * size + K * 2.0 ** -149)[fin]).all()
+
+
+@pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
+def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
+    """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
+    M, N, K, v = 16, 16, 32, 10
+    ld = 1 << 25 if dim else 1 << 23          # 16 k, or 128 rows: past 2^31 bytes
+    r = rng(77)
+    a = r.standard_normal((K, M) if ta else (M, K)).astype(np.float32)
+    b = r.standard_normal((K, N) if not tb else (N, K)).astype(np.float32)
+    X = torch.zeros((a.shape[0] - 1) * ld + a.shape[1], device="cuda")
+    for i in range(a.shape[0]):
+        X[i * ld: i * ld + a.shape[1]].copy_(torch.from_numpy(a[i]))
+    B, Cm = dev(b), torch.full((M, N), 7.0, device="cuda")
+    count = torch.tensor([v], device="cuda")
+    call("ember_gemm_f32_dyn", ta, tb, M, N, K, 1.0, p(X), ld, p(B), b.shape[1], 0.0, p(Cm), N,
+         p(count), 0, dim, None, 0, None)
+    k = 16 if dim else K                      # v rounded up to whole 16s
+    want = O.matmul(a[:k] if ta else a, b[:k] if dim else b, bool(ta), bool(tb))
+    assert_close(host(Cm), want, name="gemm dyn")
+    del X
+    torch.cuda.empty_cache()
+
+
 def test_gemm_add_rejects_overlap_and_short_rows():
     A = empty((64, 32))
     buf = empty((65, 64))
