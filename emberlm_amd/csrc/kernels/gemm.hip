@@ -338,13 +338,13 @@ struct SplitWork {  // four k of one row on their way from fp32 to three parts
 // of 512 contiguous bytes per half; the halves lie 128 bytes apart modulo the
 // 64 banks, so that the stores of four k per lane meet no bank twice.
 //   K-contiguous: lane = (row, k quad), slot = row.
-//   MN-contiguous: a wave takes one k quad; a lane takes P = ROWS / 64
-//     consecutive rows of each of its four k, and row P l + i goes to slot
-//     32 P (l / 32) + 32 i + l % 32, so that a lane's rows land in the P
-//     32-slot tiles of one wave at the same place.
-template <bool KC, int ROWS>
+//   MN-contiguous: a wave takes one k quad of 64 P rows, P = 4 ROWS / THREADS;
+//     a lane takes P consecutive rows of each of its four k, and row P l + i
+//     goes to slot 32 P (l / 32) + 32 i + l % 32, so that a lane's rows land in
+//     the P 32-slot tiles of one wave at the same place.
+template <bool KC, int ROWS, int THREADS>
 struct SplitTile {
-  static constexpr int P = ROWS / 64;
+  static constexpr int P = 4 * ROWS / THREADS;
   static constexpr int kHalf = ROWS * 16 + 128;   // bytes
   static constexpr int kPlane = 2 * kHalf;
   static constexpr int kBytes = 3 * kPlane;
@@ -354,7 +354,7 @@ struct SplitTile {
   int voff;              // this lane's first element, bytes from base
   int soff[KC ? P : 4];  // uniform offsets of the lane's loads
   int woff;              // where the lane's first four k go in LDS
-  using Vec = std::conditional_t<KC || P == 4, f32x4, f32x2>;
+  using Vec = std::conditional_t<KC || P == 4, f32x4, std::conditional_t<P == 2, f32x2, float>>;
   Vec reg[KC ? P : 4];   // K-contiguous: four k of a row; MN: P rows of a k
 
   __device__ __forceinline__ void init(const float* X, int64_t ld, int64_t R, int64_t K,
@@ -366,16 +366,17 @@ struct SplitTile {
       const int row = 16 * wave + (lane >> 2), quad = lane & 3;
       voff = static_cast<int>(row * ld * 4) + 16 * quad;
 #pragma unroll
-      for (int q = 0; q < P; ++q) soff[q] = static_cast<int>(q * 64 * ld * 4);
+      for (int q = 0; q < P; ++q) soff[q] = static_cast<int>(q * (THREADS / 4) * ld * 4);
       woff = (quad >> 1) * kHalf + row * 16 + (quad & 1) * 8;
     } else {
       base = reinterpret_cast<const char*>(X + row0);
       left = ((K - 1) * ld + R - row0) * 4;
       step = 64 * ld;
-      voff = 4 * P * lane;
+      const int quad = wave & 3, first = 64 * P * (wave >> 2);  // first row of the wave's
+      voff = 4 * (first + P * lane);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) soff[j] = static_cast<int>((4 * wave + j) * ld * 4);
-      woff = (wave >> 1) * kHalf + (32 * P * (lane >> 5) + (lane & 31)) * 16 + (wave & 1) * 8;
+      for (int j = 0; j < 4; ++j) soff[j] = static_cast<int>((4 * quad + j) * ld * 4);
+      woff = (quad >> 1) * kHalf + (first + 32 * P * (lane >> 5) + (lane & 31)) * 16 + (quad & 1) * 8;
     }
   }
 
@@ -388,12 +389,13 @@ struct SplitTile {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char*>(base), 0, static_cast<int>(min(max(left, int64_t{0}), int64_t{0x7fffffff})),
         0x00020000);
+    const int at = voff + soff[q];
     if constexpr (sizeof(Vec) == 16)
-      reg[q] =
-          __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b128(rs, voff + soff[q], 0, 0));
+      reg[q] = __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
+    else if constexpr (sizeof(Vec) == 8)
+      reg[q] = __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
     else
-      reg[q] =
-          __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b64(rs, voff + soff[q], 0, 0));
+      reg[q] = __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0));
 #endif
   }
   __device__ __forceinline__ void next() {
@@ -407,7 +409,9 @@ struct SplitTile {
   }
   // Element (k j of the lane's quad, row i of the lane's P).
   __device__ __forceinline__ float at(int j, int i) const {
-    return KC ? reg[i][j] : reg[j][i];
+    if constexpr (KC) return reg[i][j];
+    else if constexpr (P == 1) return reg[j];
+    else return reg[j][i];
   }
   // The split of row i's four k, in kSteps steps of at most four VALU
   // operations for the spaces between MFMAs; the last stores the parts.
@@ -437,7 +441,7 @@ struct SplitTile {
       w.part[2] = u32x2{pack_bf16(w.x[0], w.x[1]), pack_bf16(w.x[2], w.x[3])};
 #pragma unroll
       for (int p = 0; p < 3; ++p)
-        *reinterpret_cast<u32x2*>(lds + woff + p * kPlane + i * (KC ? 64 : 32) * 16) = w.part[p];
+        *reinterpret_cast<u32x2*>(lds + woff + p * kPlane + i * (KC ? THREADS / 4 : 32) * 16) = w.part[p];
     }
   }
   template <bool FLIP, bool MASK>
@@ -486,17 +490,18 @@ __device__ __forceinline__ unsigned out_of_range(unsigned bits) {
   return (bits << 1) + (0u - 2 * kSmall);
 }
 
-// 256 threads = 4 waves in 2x2, wave tiles (BM/2)x(BN/2); LDS is double
-// buffered.  A 256x256 block has a CU to itself and one wave per SIMD, so the
+// THREADS = 256: 4 waves in 2x2, wave tiles (BM/2)x(BN/2); 512: 8 waves in
+// 4x2.  LDS is double buffered.  A 256x256 block has a CU to itself and one wave per SIMD, so the
 // order of the wave's own instructions is what keeps the matrix core busy:
 // it is written out MFMA by MFMA and pinned (sched_barrier), two to eight
 // VALU operations of the split between two MFMAs of 32 cycles each.  Left to
 // the compiler, the same work ran at 207 TFLOP/s instead of 241.
-template <bool A_KC, bool B_KC, int BM, int BN, int OCC, bool TAIL>
-__global__ __launch_bounds__(kThreads, OCC) void gemm_f32_split(GemmArgs a) {
-  using TA = SplitTile<A_KC, BM>;
-  using TB = SplitTile<B_KC, BN>;
-  constexpr int FI = BM / 64, FJ = BN / 64;
+template <bool A_KC, bool B_KC, int BM, int BN, int THREADS, int OCC, bool TAIL>
+__global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
+  using TA = SplitTile<A_KC, BM, THREADS>;
+  using TB = SplitTile<B_KC, BN, THREADS>;
+  constexpr int kWM = THREADS / 128;                     // waves along M; two along N
+  constexpr int FI = BM / (32 * kWM), FJ = BN / 64;      // 32x32 tiles per wave
   constexpr int kStage = TA::kBytes + TB::kBytes;
   __shared__ __attribute__((aligned(256))) char lds[2 * kStage];
 
@@ -532,7 +537,7 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_split(GemmArgs a) {
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
   const int64_t nk = (K + 15) / 16;
-  const int ra = g * TA::kHalf + (wm * (BM / 2) + r) * 16;
+  const int ra = g * TA::kHalf + (wm * (BM / kWM) + r) * 16;
   const int rb = TA::kBytes + g * TB::kHalf + (wn * (BN / 2) + r) * 16;
   const unsigned start = (__builtin_popcountll(bz) & 1) ? 0x80000000u : 0u;
   if (nk > 0) {
@@ -571,7 +576,11 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_split(GemmArgs a) {
     auto stage = [&](auto odd) {
       constexpr int kOdd = decltype(odd)::value;
       constexpr int kGroup = 6 * FJ;
-      constexpr int kSlots = (FI - 1) * kGroup - (FI > 2 ? 8 : 2);  // for the splits
+      // MFMA slots: the barrier's, those for the splits, fragment reads per
+      // slot after the barrier.
+      constexpr int kTurn = FI > 1 ? (FI - 1) * kGroup : 8;
+      constexpr int kSlots = kTurn - (FI > 2 ? 8 : FI > 1 ? 2 : 1);
+      constexpr int kReads = FI > 1 ? 1 : 3;
       constexpr int kQuads = TA::P + TB::P;
       constexpr int kWork = kQuads * TA::kSteps;
       const char* cur = lds + kOdd * kStage;
@@ -586,17 +595,22 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_split(GemmArgs a) {
 #pragma unroll
           for (int j = 0; j < FJ; ++j) {
             const int in = t * FJ + j, m = i * kGroup + in;
-            if (i == FI - 1 && in == 0) {
+            if (m == kTurn) {
               wait_lgkm0();
               block_barrier();
             }
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                fa[i & 1][pa[t]], fb[kOdd][j][pb[t]], acc[i][j], 0, 0, 0);
-            if (i < FI - 1) {
-              if (in < 3) fa[(i + 1) & 1][in] = TA::frag(cur, ra, in, i + 1);
-            } else if (in < 3 + 3 * FJ) {
-              if (in < 3) fa[0][in] = TA::frag(nxt, ra, in, 0);
-              else fb[1 - kOdd][(in - 3) / 3][(in - 3) % 3] = TB::frag(nxt, rb, (in - 3) % 3, (in - 3) / 3);
+                fa[FI > 1 ? i & 1 : kOdd][pa[t]], fb[kOdd][j][pb[t]], acc[i][j], 0, 0, 0);
+            if (i < FI - 1 && in < 3) fa[(i + 1) & 1][in] = TA::frag(cur, ra, in, i + 1);
+            if (m >= kTurn) {
+#pragma unroll
+              for (int f = (m - kTurn) * kReads; f < (m - kTurn + 1) * kReads; ++f) {
+                if (f < 3)
+                  fa[FI > 1 ? 0 : 1 - kOdd][f] = TA::frag(nxt, ra, f, 0);
+                else if (f < 3 + 3 * FJ)
+                  fb[1 - kOdd][(f - 3) / 3][(f - 3) % 3] =
+                      TB::frag(nxt, rb, (f - 3) % 3, (f - 3) / 3);
+              }
             }
             if (m < kSlots) {
 #pragma unroll
@@ -634,14 +648,14 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_split(GemmArgs a) {
 
   // The lane's place in the output: register e of tile (i, j) is row slot
   // x = 8 (e / 4) + 4 g + e % 4 of MFMA tile i and column slot r of tile j.
-  const int64_t rw0 = m0 + wm * (BM / 2), cw0 = n0 + wn * (BN / 2);
+  const int64_t rw0 = m0 + wm * (BM / kWM), cw0 = n0 + wn * (BN / 2);
   if (rw0 >= a.M || cw0 >= a.N) return;
   const auto row_of = [&](int i, int e) {  // its uniform part; the lane's is lrow
     const int x = 8 * (e >> 2) + (e & 3);
-    return A_KC ? i * 32 + x : FI * x + i;
+    return A_KC || TA::P == 1 ? i * 32 + x : FI * x + i;
   };
-  const auto col_of = [&](int j) { return B_KC ? j * 32 + r : FJ * r + j; };
-  const int lrow = A_KC ? 4 * g : FI * 4 * g;
+  const auto col_of = [&](int j) { return B_KC || TB::P == 1 ? j * 32 + r : FJ * r + j; };
+  const int lrow = A_KC || TA::P == 1 ? 4 * g : FI * 4 * g;
   const int rows_left = static_cast<int>(min(a.M - rw0, int64_t{BM}));
   const int cols_left = static_cast<int>(min(a.N - cw0, int64_t{BN}));
 
@@ -673,7 +687,7 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_split(GemmArgs a) {
     // This wave's tile in fp32 from global memory, 32x32 at a time.
     for (int t = 0; t < FI * FJ; ++t) {
       const int i = t / FJ, j = t % FJ;
-      const int64_t ar = min(rw0 + (A_KC ? i * 32 + r : FI * r + i), a.M - 1);
+      const int64_t ar = min(rw0 + (A_KC || TA::P == 1 ? i * 32 + r : FI * r + i), a.M - 1);
       const int64_t bc = min(cw0 + col_of(j), a.N - 1);
       const float* pa = A_KC ? A + ar * a.lda : A + ar;
       const float* pb = B_KC ? B + bc * a.ldb : B + bc;
@@ -741,7 +755,7 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_split(GemmArgs a) {
       }
     }
   };
-  const bool full = rows_left >= BM / 2;
+  const bool full = rows_left >= BM / kWM;
   if (a.beta != 0.f) {
     if (full) store_all(std::false_type{}, std::true_type{});
     else store_all(std::true_type{}, std::true_type{});
@@ -947,9 +961,14 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
 // round `ends` more for its first loads and its stores, which only other
 // blocks on the same CU can cover.  A split adds its reduction: one launch
 // and S + 1 planes of C through HBM.  The constants are fitted to times of
-// 59 products (M, N 32 to 151936, K 64 to 151936, all three layouts) on every
-// tile with 1 to 16 splits; choosing by them is on average 0.5% slower than
-// the best of those, at worst 6%.
+// 45 products (M, N 32 to 151936, K 64 to 8192, three layouts) on the tiles
+// with 1 to 16 splits; choosing by them is on average 0.5% slower than the
+// best of those, at worst 4%.  The 512-thread tile is for grids of one block
+// per CU, where one wave per SIMD cannot issue fast enough (a stage alone
+// takes 0.37-0.44 us instead of 0.53: 256x576x576 13.2 -> 12.1 us,
+// 2048x576x1536 33.1 -> 29.7, 509x3072x1024 31.7 -> 28.6, 1000x2048x2048
+// 56.4 -> 52.4); with more blocks it is slower (4096x3072x1024 151 against
+// 130 us).
 struct SplitPlan {
   int tile;         // index into kTiles
   int64_t splits;   // 1 = no K split
@@ -960,8 +979,9 @@ struct TileCost {
   int per_cu;
   double stage[3], alone, ends;
 };
-constexpr TileCost kTiles[3] = {{128, 128, 3, {0.67, 1.12, 1.89}, 0.53, 3.71},
-                                {256, 128, 2, {1.11, 2.19}, 0.78, 7.0},
+constexpr TileCost kTiles[4] = {{128, 128, 1, {0.61}, 0.44, 2.8},  // 512 threads
+                                {128, 128, 3, {0.92, 1.17, 1.89}, 0.53, 4.56},
+                                {256, 128, 2, {1.16, 2.19}, 0.78, 6.01},
                                 {256, 256, 1, {1.92}, 1.38, 27.3}};
 
 double predicted_us(const TileCost& t, int64_t M, int64_t N, int64_t K, int64_t batch,
@@ -989,14 +1009,15 @@ double predicted_us(const TileCost& t, int64_t M, int64_t N, int64_t K, int64_t 
 // from 64-bit sums, and 4% faster).
 SplitPlan make_split_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t room,
                           int tiles) {
-  SplitPlan best{0, 1, 0};
+  SplitPlan best{1, 1, 0};
   double least = 1e30;
   for (int t = 0; t < tiles; ++t)
     for (int64_t s = K >= 4096 ? room : 1; s <= room; ++s) {
       const int64_t chunk = s > 1 ? cdiv(cdiv(K, s), 32) * 32 : K;
       const int64_t n = s > 1 ? cdiv(K, chunk) : 1;  // at most s
+      if (t == 0 && cdiv(M, 128) * cdiv(N, 128) * batch * n > kCUs) continue;  // one round only
       double us = predicted_us(kTiles[t], M, N, chunk, batch, n);
-      if (n > 1) us += 2.45 + static_cast<double>((n + 1) * M * N) * 4 / 5.68e6;
+      if (n > 1) us += 2.45 + static_cast<double>((n + 1) * M * N) * 4 / 5.21e6;
       if (us < least) {
         least = us;
         best = SplitPlan{t, n, n > 1 ? chunk : 0};
@@ -1025,7 +1046,7 @@ int launch_t(GemmArgs a, bool a_kc, bool b_kc, int64_t ny, bool vec, hipStream_t
   return launch<false, true, BM, BN, OCC>(a, ny, vec, st);
 }
 
-template <bool A_KC, bool B_KC, int BM, int BN, int OCC>
+template <bool A_KC, bool B_KC, int BM, int BN, int THREADS, int OCC>
 int launch_split_t(GemmArgs a, int64_t ny, hipStream_t st) {
   a.tiles_m = static_cast<int>(cdiv(a.M, BM));
   a.tiles_n = static_cast<int>(cdiv(a.N, BN));
@@ -1035,24 +1056,25 @@ int launch_split_t(GemmArgs a, int64_t ny, hipStream_t st) {
   const bool whole = (a.kchunk > 0 ? a.kchunk : a.K) % 32 == 0 && a.K % 32 == 0 &&
                      !(a.dyn && a.dyn_dim == 1);
   if ((A_KC || B_KC) && !whole)
-    gemm_f32_split<A_KC, B_KC, BM, BN, OCC, true><<<grid, kThreads, 0, st>>>(a);
+    gemm_f32_split<A_KC, B_KC, BM, BN, THREADS, OCC, true><<<grid, THREADS, 0, st>>>(a);
   else
-    gemm_f32_split<A_KC, B_KC, BM, BN, OCC, false><<<grid, kThreads, 0, st>>>(a);
+    gemm_f32_split<A_KC, B_KC, BM, BN, THREADS, OCC, false><<<grid, THREADS, 0, st>>>(a);
   return launch_status();
 }
 
-template <int BM, int BN, int OCC>
+template <int BM, int BN, int THREADS, int OCC>
 int launch_split_tile(const GemmArgs& a, bool a_kc, bool b_kc, int64_t ny, hipStream_t st) {
-  if (a_kc && b_kc) return launch_split_t<true, true, BM, BN, OCC>(a, ny, st);
-  if (a_kc && !b_kc) return launch_split_t<true, false, BM, BN, OCC>(a, ny, st);
-  if (!a_kc && !b_kc) return launch_split_t<false, false, BM, BN, OCC>(a, ny, st);
-  return launch_split_t<false, true, BM, BN, OCC>(a, ny, st);
+  if (a_kc && b_kc) return launch_split_t<true, true, BM, BN, THREADS, OCC>(a, ny, st);
+  if (a_kc && !b_kc) return launch_split_t<true, false, BM, BN, THREADS, OCC>(a, ny, st);
+  if (!a_kc && !b_kc) return launch_split_t<false, false, BM, BN, THREADS, OCC>(a, ny, st);
+  return launch_split_t<false, true, BM, BN, THREADS, OCC>(a, ny, st);
 }
 
 int launch_split(const GemmArgs& a, int tile, bool a_kc, bool b_kc, int64_t ny, hipStream_t st) {
-  return tile == 0   ? launch_split_tile<128, 128, 3>(a, a_kc, b_kc, ny, st)
-         : tile == 1 ? launch_split_tile<256, 128, 2>(a, a_kc, b_kc, ny, st)
-                     : launch_split_tile<256, 256, 1>(a, a_kc, b_kc, ny, st);
+  return tile == 0   ? launch_split_tile<128, 128, 512, 2>(a, a_kc, b_kc, ny, st)
+         : tile == 1 ? launch_split_tile<128, 128, 256, 3>(a, a_kc, b_kc, ny, st)
+         : tile == 2 ? launch_split_tile<256, 128, 256, 2>(a, a_kc, b_kc, ny, st)
+                     : launch_split_tile<256, 256, 256, 1>(a, a_kc, b_kc, ny, st);
 }
 
 // How many of kTiles gemm_f32_split can use for these operands: none unless
@@ -1067,7 +1089,7 @@ int split_tiles(const GemmArgs& a, bool a_kc, bool b_kc, bool vec) {
     return (a_kc ? rows - 1 : 16) * a.lda < top && (b_kc ? rows - 1 : 16) * a.ldb < top &&
            rows * std::max(a.ldc, a.D ? a.ldd : int64_t{0}) < top;
   };
-  return fits(256) ? 3 : fits(128) ? 1 : 0;
+  return fits(256) ? 4 : fits(128) ? 2 : 0;
 }
 
 int check_args(int transa, int transb, int64_t M, int64_t N, int64_t K, const float* A,

@@ -758,6 +758,7 @@ def _gemm_dev(A, B, ta, tb, M, N, K, ws=True, beta=0.0, c=None):
 @pytest.mark.parametrize("M,N,K", [
     (12, 16, 4), (128, 128, 16), (132, 260, 36),      # 128x128: one tile, edges, k past a stage
     (4, 4, 100), (500, 124, 1000),                    # few tiles: K splits, odd last chunk
+    (2048, 2048, 100), (2048, 2052, 40), (4096, 2048, 64),  # 256, 272, 512 tiles of 128x128
     (4092, 2052, 260), (4096, 4096, 48),              # larger tiles, ragged and whole, odd stages
     (8196, 2564, 224),
 ])
