@@ -33,7 +33,7 @@
 //                the KV head's group, in a fixed order.  With a dS buffer it
 //                also stores dS (fp32, the causal part only, see below);
 //   attn_bwd_dq_gemm: dQ = dS K from the stored dS, a plain product in key
-//                order on the GEMM kernel's 256 x D tiles;
+//                order on 256 x D tiles;
 //   attn_bwd_dq (no dS buffer): per 16 queries, S^T = K Q^T and dP^T =
 //                V dO^T recomputed, then dQ^T += K^T dS^T.
 // Counted in units of one T x T x D product per head, the algorithm needs 4
@@ -792,15 +792,14 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dkdv_kernel(
   }
 }
 
-// dQ = scale * dS K from the stored dS on the GEMM kernel's machinery
-// (gemm.hip's gemm_f32_dma): m = query, n = d, contraction over keys; 256
+// dQ = scale * dS K from the stored dS as an fp32 GEMM staged by DMA: m =
+// query, n = d, contraction over keys; 256
 // queries x D per workgroup, four waves in 2 x 2 on v_mfma_f32_32x32x2f32
 // tiles; 16-key stages copied global -> LDS by global_load_lds_dwordx4 into a
 // 3-stage ring two stages ahead of the MFMAs, up to the tile's last query.
 //   A = dS^T: a key's row of its strip holds queries 64 sb ... contiguously,
 //     so one 1 KB DMA block is one key's 256 queries (chunk q of key row k at
-//     chunk position q ^ (8 ((k >> 2) & 1)), as the GEMM lays out an
-//     M-contiguous tile), read back as b128 rows of four consecutive queries.
+//     chunk position q ^ (8 ((k >> 2) & 1))), read back as b128 rows of four consecutive queries.
 //   B = K rows (d contiguous), laid out the same way.
 // Entries with query < key are zeroed in registers after the LDS read: the
 // dK/dV kernel does not write all of them, and a tile's queries before a
@@ -945,7 +944,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_gemm_kernel(
   load_a(lds, 0, 0, fa0);
   load_b(lds, 0, fb0);
 
-  // The GEMM kernel's stage: slab 1's reads, slab 0's MFMAs with them spread
+  // A stage: slab 1's reads, slab 0's MFMAs with them spread
   // among, the DMA two stages ahead, slab 1's first MFMAs, the barrier after
   // stage kt+1's copy has landed, the next stage's slab-0 reads under slab
   // 1's last MFMAs.
