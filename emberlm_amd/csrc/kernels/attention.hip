@@ -225,7 +225,8 @@ __device__ __forceinline__ float sum_over_rows(float x) {
 }
 
 // ------------------------------------------------------------------ forward
-// Forward.  A wave owns 16 queries and a workgroup of eight waves 128, so
+// Forward.  A wave owns 16 queries and a workgroup of eight waves 128 (or of
+// four 64, below), so
 // every K/V tile in LDS serves 128 queries, and at 100 registers per lane
 // (D = 128) four waves fit on a SIMD (32 queries per wave on 32x32x2 tiles
 // took 239 and two waves: 1.14x slower at B=8, T=4096, H=16, Hk=8).  K and V
@@ -243,9 +244,15 @@ __device__ __forceinline__ float sum_over_rows(float x) {
 //   LDS read of V (d = 64hq + 4i .. +3) feeds the four tiles 4hq .. 4hq + 3.
 //   Each element of O sums the same products in the same order as with
 //   d = 16t + x; only its register moves.
-template <int D>
+//
+// A wave's MFMAs of one tile take 4096 cycles at D = 128, and the last query
+// block has T / 32 tiles in a row.  While blocks of 128 queries are at most
+// one per CU (fwd_queries), blocks are of 64 queries and four waves instead:
+// with one wave per SIMD that row runs up to twice as fast, on CUs that were
+// idle; L2 serves twice the K/V copies per query.  A wave's sums are the same.
+template <int D, int BQ>
 struct FwdCfg {
-  static constexpr int kThreads = 512, kBQ = 128, kBK = 32;
+  static constexpr int kThreads = 4 * BQ, kBQ = BQ, kBK = 32;
   using Tile = DmaTile<D, kBK, kThreads / 64>;
   static constexpr int kTile = Tile::kFloats;
   static constexpr int kBuf = 2 * kTile;  // one K+V stage
@@ -255,12 +262,12 @@ struct FwdCfg {
 // SS: also store every computed score (log2 units, before the mask) in the
 // dS layout of the KV row's region given by `s_rows` (attn_bwd_from_scores
 // reads them back instead of computing S again).
-template <int D, bool SS>
-__global__ __launch_bounds__(FwdCfg<D>::kThreads, 2) void attn_fwd_kernel(
+template <int D, int BQ, bool SS>
+__global__ __launch_bounds__(4 * BQ, 2) void attn_fwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     float* __restrict__ o, float* __restrict__ lse, float* const* __restrict__ s_rows, int T,
     int H, int Hk, float scale_log2) {
-  using C = FwdCfg<D>;
+  using C = FwdCfg<D, BQ>;
   constexpr int NT = D / 16;
   __shared__ __attribute__((aligned(16))) float smem[C::kSmem];
 
@@ -1023,9 +1030,43 @@ int check_shapes(int64_t B, int64_t T, int64_t H, int64_t Hk, int64_t D) {
   if (B < 0 || T < 0 || H <= 0 || Hk <= 0 || H % Hk != 0) return EMBER_EINVAL;
   if (D != 64 && D != 128) return EMBER_EINVAL;
   if (T > 0x7fffffff / 2 || H > 65535 || Hk > 65535 || B > 65535) return EMBER_EINVAL;
-  // 1-D grids: 128-query forward tiles, 64-row backward tiles, Hk <= H.
+  // 1-D grids: 128- or 64-query forward tiles, 64-row backward tiles, Hk <= H.
   if ((T + 63) / 64 * H * B > 0x7fffffff) return EMBER_EINVAL;
   return EMBER_OK;
+}
+
+}  // namespace
+
+namespace {
+
+// Queries per block of the forward: 64 where blocks of 128 are at most one
+// per CU.  In us, with 128 -> with 64 (B T H Hk D): 1 128 16 8 128 18.9 ->
+// 13.1, 1 509 16 8 128 67.7 -> 40.7, 1 1024 16 8 128 133 -> 77, 1 512 9 3 64
+// 37.2 -> 23.0; at exactly 256 blocks 1 2048 16 8 128 262 -> 202, 1 1000 32 8
+// 64 74.1 -> 59.4 (causal blocks differ in length, so halves pack better).
+constexpr int64_t kCUs = 256;
+int fwd_queries(int64_t B, int64_t T, int64_t H) {
+  return (T + 127) / 128 * H * B <= kCUs ? 64 : 128;
+}
+
+template <int D, int BQ, bool SS>
+void launch_fwd_t(const float* q, const float* k, const float* v, float* o, float* lse,
+                  float* const* s_rows, int64_t B, int64_t T, int64_t H, int64_t Hk, float scale,
+                  hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>((T + BQ - 1) / BQ * H * B));
+  attn_fwd_kernel<D, BQ, SS><<<grid, FwdCfg<D, BQ>::kThreads, 0, st>>>(
+      q, k, v, o, lse, s_rows, static_cast<int>(T), static_cast<int>(H), static_cast<int>(Hk),
+      scale * kLog2e);
+}
+
+template <bool SS>
+void launch_fwd(const float* q, const float* k, const float* v, float* o, float* lse,
+                float* const* s_rows, int64_t B, int64_t T, int64_t H, int64_t Hk, int64_t D,
+                float scale, hipStream_t st) {
+  const bool small = fwd_queries(B, T, H) == 64;
+  auto run = D == 64 ? (small ? launch_fwd_t<64, 64, SS> : launch_fwd_t<64, 128, SS>)
+                     : (small ? launch_fwd_t<128, 64, SS> : launch_fwd_t<128, 128, SS>);
+  run(q, k, v, o, lse, s_rows, B, T, H, Hk, scale, st);
 }
 
 }  // namespace
@@ -1038,16 +1079,7 @@ extern "C" int ember_attn_fwd(const float* q, const float* k, const float* v, fl
   if (B == 0 || T == 0) return EMBER_OK;
   if (!q || !k || !v || !o || !lse) return EMBER_EINVAL;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o)) return EMBER_EALIGN;
-  static_assert(FwdCfg<64>::kBQ == 128 && FwdCfg<128>::kBQ == 128, "grid assumes 128 queries");
-  const dim3 grid(static_cast<unsigned>((T + 127) / 128 * H * B));
-  const float sl = scale * kLog2e;
-  const int Ti = static_cast<int>(T), Hi = static_cast<int>(H), Hki = static_cast<int>(Hk);
-  if (D == 64)
-    attn_fwd_kernel<64, false><<<grid, FwdCfg<64>::kThreads, 0, as_stream(s)>>>(
-        q, k, v, o, lse, nullptr, Ti, Hi, Hki, sl);
-  else
-    attn_fwd_kernel<128, false><<<grid, FwdCfg<128>::kThreads, 0, as_stream(s)>>>(
-        q, k, v, o, lse, nullptr, Ti, Hi, Hki, sl);
+  launch_fwd<false>(q, k, v, o, lse, nullptr, B, T, H, Hk, D, scale, as_stream(s));
   return launch_status();
 }
 
@@ -1265,15 +1297,7 @@ extern "C" int ember_attn_fwd_scores(const float* q, const float* k, const float
   float** table = static_cast<float**>(workspace);
   if ((rc = upload_async(table, host_table.data(), host_table.size() * sizeof(float*), st)))
     return rc;
-  const dim3 grid(static_cast<unsigned>((T + 127) / 128 * H * B));
-  const float sl = scale * kLog2e;
-  const int Ti = static_cast<int>(T), Hi = static_cast<int>(H), Hki = static_cast<int>(Hk);
-  if (D == 64)
-    attn_fwd_kernel<64, true><<<grid, FwdCfg<64>::kThreads, 0, st>>>(q, k, v, o, lse, table, Ti,
-                                                                      Hi, Hki, sl);
-  else
-    attn_fwd_kernel<128, true><<<grid, FwdCfg<128>::kThreads, 0, st>>>(q, k, v, o, lse, table, Ti,
-                                                                        Hi, Hki, sl);
+  launch_fwd<true>(q, k, v, o, lse, table, B, T, H, Hk, D, scale, st);
   return launch_status();
 }
 

@@ -1145,6 +1145,34 @@ def test_attention_fwd_bwd_vs_oracle(B, T, H, Hk, D):
     assert torch.equal(DQ, DQ2) and torch.equal(DK, DK2) and torch.equal(DV, DV2)
 
 
+@pytest.mark.parametrize("T,H,Hk,D", [
+    (1, 4, 2, 128), (16, 8, 8, 64), (63, 8, 4, 128), (65, 4, 4, 64), (128, 8, 2, 128),
+    (129, 4, 1, 64), (300, 8, 4, 128),
+])
+def test_attention_fwd_block_sizes_agree(T, H, Hk, D):
+    """Grids of at most 256 blocks of 128 queries run on 64-query blocks: both,
+    and with the scores kept, give a sequence the same bits."""
+    r = rng(T + H + D)
+    q, k, v = (r.standard_normal((1, T, n, D)).astype(np.float32) for n in (H, Hk, Hk))
+    scale = 1.0 / math.sqrt(D)
+    o_ref, lse_ref = O.attention_fwd(q, k, v, scale)
+    row = capi.lib().ember_attn_bwd_ds_row_bytes(T, H, Hk)
+    per = -(-T // 128) * H  # 128-query blocks of one sequence
+    first = None
+    for B in (1, 256 // per, 256 // per + 1):
+        Q, K, Vv = (dev(np.repeat(x, B, 0)) for x in (q, k, v))
+        Ot, L = empty((B, T, H, D)), empty((B, H, T))
+        call("ember_attn_fwd", p(Q), p(K), p(Vv), p(Ot), p(L), B, T, H, Hk, D, scale, None)
+        if first is None:
+            first = Ot, L
+            assert_close(host(Ot), o_ref, name="attn o")
+            assert_close(host(L), lse_ref, name="attn lse")
+        kept = _keep_scores_run(Q, K, Vv, Q, B, T, H, Hk, D, scale, [B * Hk * row])[:2]
+        for got in ((Ot, L), kept):
+            for x, want in zip(got, first):
+                assert torch.equal(x, want.expand_as(x))
+
+
 def _attn_hip(Q, K, Vv, DO, B, T, H, Hk, D, scale, wsb=None):
     """Forward and backward through the C ABI on device tensors (the backward
     with `wsb` bytes of workspace, by default all it can use)."""
