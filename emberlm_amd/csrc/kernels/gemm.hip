@@ -482,6 +482,8 @@ struct SplitTile {
 // range, has no three parts (the result is then not finite), and below 2^-110
 // the last part runs out of exponent.  Such a result, not finite or below
 // 2^-100, is found here and taken again in fp32.
+// (A factor y of a value below 2^-110 may add an error of 2^-134 |y| to a
+// larger result: below fp32's own rounding unless |y| is over 2^110 times it.)
 // `out_of_range` of a value's bits: at least kOutOfRange for such a value and
 // for a zero, which is told apart only when one of these is there.
 constexpr unsigned kSmall = 0x0d800000u, kInf = 0x7f800000u;  // 2^-100, infinity
