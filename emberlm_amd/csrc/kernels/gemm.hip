@@ -774,6 +774,9 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
 //   S > 0: float4s, S planes known when compiled, so that all their loads are
 //   in flight at once (in a loop, eight planes cost eight trips to memory:
 //   256x576x576 in six chunks 12.1 us, now 11.5).
+//   Splits past kMaxPlanes (a long K, as over a vocabulary: 1024x1024x32768
+//   has 32) follow in a loop.
+constexpr int kMaxPlanes = 16;
 template <int S>
 __global__ __launch_bounds__(kThreads) void splitk_reduce(const float* __restrict__ P, float* C,
                                                           int64_t M, int64_t N, int64_t ldc,
@@ -807,6 +810,14 @@ __global__ __launch_bounds__(kThreads) void splitk_reduce(const float* __restric
     for (int k = 1; k < S; ++k)
 #pragma unroll
       for (int e = 0; e < 4; ++e) s[e] += t[k][e];
+    if constexpr (S == kMaxPlanes) {  // the planes past the first kMaxPlanes
+#pragma unroll 8
+      for (int k = S; k < splits; ++k) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(P + k * plane + m * N + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += x[e];
+      }
+    }
     f32x4 out;
 #pragma unroll
     for (int e = 0; e < 4; ++e) out[e] = beta != 0.f ? alpha * s[e] + beta * old[e] : alpha * s[e];
@@ -1188,13 +1199,13 @@ int gemm_run(int transa, int transb, int64_t M, int64_t N, int64_t K, float alph
     const unsigned blocks = static_cast<unsigned>(cdiv(items, kThreads));
     const int64_t* rdyn = dyn_dim == 0 ? dyn : nullptr;
     using Reduce = decltype(&launch_reduce_n<0>);
-    constexpr Reduce kReduce[17] = {
+    constexpr Reduce kReduce[kMaxPlanes + 1] = {
         launch_reduce_n<0>,  launch_reduce_n<1>,  launch_reduce_n<2>,  launch_reduce_n<3>,
         launch_reduce_n<4>,  launch_reduce_n<5>,  launch_reduce_n<6>,  launch_reduce_n<7>,
         launch_reduce_n<8>,  launch_reduce_n<9>,  launch_reduce_n<10>, launch_reduce_n<11>,
         launch_reduce_n<12>, launch_reduce_n<13>, launch_reduce_n<14>, launch_reduce_n<15>,
         launch_reduce_n<16>};
-    kReduce[rvec ? splits : 0](blocks, static_cast<const float*>(workspace), C, M, N, ldc,
+    kReduce[rvec ? std::min<int64_t>(splits, kMaxPlanes) : 0](blocks, static_cast<const float*>(workspace), C, M, N, ldc,
                                static_cast<int>(splits), alpha, beta, rdyn, dyn_base, D, ldd, st);
     return launch_status();
   }

@@ -1103,6 +1103,23 @@ def test_sgd_exact():
         assert np.array_equal(host(P), want)
 
 
+@pytest.mark.parametrize("M,N,K", [(1024, 1024, 32768), (1024, 1020, 32768), (512, 1024, 65536)])
+def test_gemm_more_than_sixteen_k_splits(M, N, K):
+    """A long K with few tiles has more planes than the reduction keeps in
+    registers; 2^-24 sqrt(K) of the 2-norm bounds 32-bit sums in any order here."""
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    a = torch.randn(M, K, device="cuda", generator=gen)
+    b = torch.randn(K, N, device="cuda", generator=gen)
+    wsb = capi.lib().ember_gemm_f32_workspace_bytes(M, N, K, 1)
+    assert wsb > 16 * 4 * M * N
+    ws, c = empty((wsb // 4,)), empty((M, N))
+    call("ember_gemm_f32_ws", 0, 0, M, N, K, 1.0, p(a), K, 0, p(b), N, 0, 0.0, p(c), N, 0, 1, p(ws),
+         wsb, None)
+    want = a.double() @ b.double()
+    err = (c.double() - want).norm() / want.norm()
+    assert err.item() <= 2.0 ** -24 * math.sqrt(K)
+
+
 # ------------------------------------------------------------ attention
 @pytest.mark.parametrize("B,T,H,Hk,D", [
     (1, 256, 9, 3, 64),     # c1 block attention (SmolLM2 shape)
