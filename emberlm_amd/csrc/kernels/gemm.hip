@@ -327,6 +327,12 @@ __device__ __forceinline__ float bf16_hi(unsigned u) {
   return __builtin_bit_cast(float, u & 0xffff0000u);
 }
 
+// Both operands are scaled by 2^24 first (B by the sign it is summed with, too):
+// the last part of an unscaled value below 2^-110 would have no exponent left,
+// and all three of one below 2^-134 would be zero.  Scaled, every part of every
+// subnormal is a normal bf16 value.
+constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;
+
 struct SplitWork {  // four k of one row on their way from fp32 to three parts
   float x[4];
   u32x2 part[3];
@@ -415,20 +421,18 @@ struct SplitTile {
   }
   // The split of row i's four k, in kSteps steps of at most four VALU
   // operations for the spaces between MFMAs; the last stores the parts.
-  // MASK: a K-contiguous lane's k count only when `valid`.  FLIP: `sign` (0 or the sign
-  // bit) is applied first.
+  // MASK: a K-contiguous lane's k count only when `valid`.  `scale`: +-kScale.
   static constexpr int kSteps = 7;
-  template <bool FLIP, bool MASK>
+  template <bool MASK>
   __device__ __forceinline__ void split_step(SplitWork& w, int i, int step, char* lds, bool valid,
-                                             unsigned sign) const {
-    if (step == 0 || step == 3) {
-      if (step == 0) {
+                                             float scale) const {
+    if (step == 0) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float v = MASK && KC && !valid ? 0.f : at(j, i);
-          w.x[j] = FLIP ? __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ sign) : v;
-        }
+      for (int j = 0; j < 4; ++j) {
+        const float v = MASK && KC && !valid ? 0.f : at(j, i);
+        w.x[j] = v * scale;
       }
+    } else if (step == 1 || step == 3) {
       const int p = step / 3;
       w.part[p] = u32x2{pack_bf16(w.x[0], w.x[1]), pack_bf16(w.x[2], w.x[3])};
     } else if (step == 2 || step == 5) {
@@ -444,13 +448,13 @@ struct SplitTile {
         *reinterpret_cast<u32x2*>(lds + woff + p * kPlane + i * (KC ? THREADS / 4 : 32) * 16) = w.part[p];
     }
   }
-  template <bool FLIP, bool MASK>
-  __device__ __forceinline__ void store_all(char* lds, bool valid, unsigned sign) const {
+  template <bool MASK>
+  __device__ __forceinline__ void store_all(char* lds, bool valid, float scale) const {
 #pragma unroll
     for (int i = 0; i < P; ++i) {
       SplitWork w;
 #pragma unroll
-      for (int t = 0; t < kSteps; ++t) split_step<FLIP, MASK>(w, i, t, lds, valid, sign);
+      for (int t = 0; t < kSteps; ++t) split_step<MASK>(w, i, t, lds, valid, scale);
     }
   }
   // Part p of 32-slot tile t (from the wave's first), for lane offset `off`.
@@ -478,20 +482,9 @@ struct SplitTile {
 // place).  K splits start negated by the parity of the number's count of ones
 // (0 1 1 0 1 0 0 1 ...).  Turning 256 accumulators costs about one stage.
 //
-// What the split cannot give: a value that is not finite, or beyond bf16's
-// range, has no three parts (the result is then not finite), and below 2^-110
-// the last part runs out of exponent.  Such a result, not finite or below
-// 2^-100, is found here and taken again in fp32.
-// (A factor y of a value below 2^-110 may add an error of 2^-134 |y| to a
-// larger result: below fp32's own rounding unless |y| is over 2^110 times it.)
-// `out_of_range` of a value's bits: at least kOutOfRange for such a value and
-// for a zero, which is told apart only when one of these is there.
-constexpr unsigned kSmall = 0x0d800000u, kInf = 0x7f800000u;  // 2^-100, infinity
-constexpr unsigned kOutOfRange = 2 * (kInf - kSmall);
-__device__ __forceinline__ unsigned out_of_range(unsigned bits) {
-  return (bits << 1) + (0u - 2 * kSmall);
-}
-
+// What the split cannot give: an infinity or NaN has no three parts, nor has a
+// value of 2^104 or more once scaled; such a result, or one past 2^80, is not
+// finite, which is found here, and it is taken again in fp32.
 // THREADS = 256: 4 waves in 2x2, wave tiles (BM/2)x(BN/2); 512: 8 waves in
 // 4x2.  LDS is double buffered.  A 256x256 block has a CU to itself and one wave per SIMD, so the
 // order of the wave's own instructions is what keeps the matrix core busy:
@@ -541,13 +534,13 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   const int64_t nk = (K + 15) / 16;
   const int ra = g * TA::kHalf + (wm * (BM / kWM) + r) * 16;
   const int rb = TA::kBytes + g * TB::kHalf + (wn * (BN / 2) + r) * 16;
-  const unsigned start = (__builtin_popcountll(bz) & 1) ? 0x80000000u : 0u;
+  const bool start = __builtin_popcountll(bz) & 1;  // negated
   if (nk > 0) {
     const int64_t pairs = (nk + 1) / 2;  // an odd nk's last stage is all zeros
     const int64_t turn[3] = {(pairs * 212) >> 10, (pairs * 724) >> 10, pairs};
-    unsigned sign;  // of the values stored, which belong to pair `at`
+    float scale_b;  // of the values stored, which belong to pair `at`
     const auto sign_at = [&](int64_t at) {
-      sign = start ^ (at >= turn[0] && at < turn[1] ? 0x80000000u : 0u);
+      scale_b = start != (at >= turn[0] && at < turn[1]) ? -kScale : kScale;
     };
     sign_at(0);
     TA ta;
@@ -557,8 +550,8 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
     int64_t klane = K - 4 * (lane & 3);  // TAIL: k left from this lane's quad on
     ta.load_all();
     tb.load_all();
-    ta.template store_all<false, TAIL>(lds, klane > 0, sign);
-    tb.template store_all<true, TAIL>(lds + TA::kBytes, klane > 0, sign);
+    ta.template store_all<TAIL>(lds, klane > 0, kScale);
+    tb.template store_all<TAIL>(lds + TA::kBytes, klane > 0, scale_b);
     ta.load_all();
     tb.load_all();
     wait_lgkm0();
@@ -619,10 +612,10 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
               for (int s = m * kWork / kSlots; s < (m + 1) * kWork / kSlots; ++s) {
                 const int q = s / TA::kSteps, st = s % TA::kSteps;
                 if (q < TA::P)
-                  ta.template split_step<false, TAIL>(w, q, st, nxt, klane > 0, sign);
+                  ta.template split_step<TAIL>(w, q, st, nxt, klane > 0, kScale);
                 else
-                  tb.template split_step<true, TAIL>(w, q - TA::P, st, nxt + TA::kBytes,
-                                                     klane > 0, sign);
+                  tb.template split_step<TAIL>(w, q - TA::P, st, nxt + TA::kBytes, klane > 0,
+                                               scale_b);
                 if (s == TA::P * TA::kSteps - 1) ta.load_all();
                 if (s == kWork - 1) tb.load_all();
               }
@@ -661,31 +654,14 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   const int rows_left = static_cast<int>(min(a.M - rw0, int64_t{BM}));
   const int cols_left = static_cast<int>(min(a.N - cw0, int64_t{BN}));
 
-  // (Values are taken out before their bits: a bit_cast of a vector element
-  // reads element 0.)
-  unsigned most = 0;
+  float bad = 0.f;  // NaN once some value is not finite
 #pragma unroll
   for (int i = 0; i < FI; ++i)
 #pragma unroll
     for (int j = 0; j < FJ; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float f = acc[i][j][e];
-        most = max(most, out_of_range(__builtin_bit_cast(unsigned, f)));
-      }
-  bool redo = false;
-  if (__any(most >= kOutOfRange)) {
-#pragma unroll
-    for (int i = 0; i < FI; ++i)
-#pragma unroll
-      for (int j = 0; j < FJ; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float f = acc[i][j][e];
-          redo |= f != 0.f && out_of_range(__builtin_bit_cast(unsigned, f)) >= kOutOfRange;
-        }
-  }
-  if (__builtin_expect(__any(redo), 0)) {
+      for (int e = 0; e < 16; ++e) bad = __builtin_fmaf(acc[i][j][e], 0.f, bad);
+  if (__builtin_expect(__any(bad != bad), 0)) {
     // This wave's tile in fp32 from global memory, 32x32 at a time.
     for (int t = 0; t < FI * FJ; ++t) {
       const int i = t / FJ, j = t % FJ;
@@ -714,7 +690,7 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
     return;
   }
 
-  const float back = start ? -1.f : 1.f;
+  const float back = start ? -kUnscale : kUnscale;
 #if defined(__HIP_DEVICE_COMPILE__)
   // Stores (and the beta term's loads) through buffer resources based at this
   // wave's first output row of C (and of D): a row's byte offset splits into a

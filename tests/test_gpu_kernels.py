@@ -818,7 +818,9 @@ def test_gemm_split_nonfinite_and_range(ta, tb, M, N, K):
     a[11, 0] = 3.4e38                       # rounds to infinity in bf16
     a[13] = 0.0
     a[13, 0] = a[13, 2] = 3e38              # overflows
-    a[15] *= 2.0 ** -120                    # the last part of the split has no exponent left
+    a[15] *= 2.0 ** -120
+    a[19] = 0.0
+    a[19, 0] = 2.0 ** 110                   # scaled by 2^24, past bf16's largest
     a[17] = 0.0
     b[21] *= 2.0 ** -130
     A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
@@ -834,6 +836,30 @@ def test_gemm_split_nonfinite_and_range(ta, tb, M, N, K):
     size = a.double().abs().masked_fill(~torch.isfinite(a), 0) @ b.double().t().contiguous()
     # fp32 sums of K terms, and the smallest subnormal per term
     assert ((got.double() - ref).abs()[fin] <= (K * 2.0 ** -24 * size + K * 2.0 ** -149)[fin]).all()
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("small_is_a", [True, False])
+@pytest.mark.parametrize("M,N,K,t", [(140, 132, 52, 100), (2048, 2048, 64, 100),
+                                     (4096, 4096, 64, 100), (140, 132, 52, 0)])
+def test_gemm_split_small_operands(ta, tb, small_is_a, M, N, K, t):
+    """Operands down to the smallest subnormal count in full: rows (columns) of values near
+    2^-100 ... 2^-149 against values near 2^100, where the results are ordinary numbers,
+    and near 1.  Bound: fp32 sums of K terms, and of a smallest subnormal each."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    R, S = (M, N) if small_is_a else (N, M)
+    x = torch.randn(R, K, device="cuda", generator=g)
+    x *= torch.exp2(-100.0 - torch.arange(R, device="cuda") % 50)[:, None]
+    x[0] = 2.0 ** -149
+    y = torch.randn(S, K, device="cuda", generator=g) * 2.0 ** t
+    ref = x.double() @ y.double().t().contiguous()
+    size = x.double().abs() @ y.double().abs().t().contiguous()
+    a, b = (x, y) if small_is_a else (y, x)
+    if not small_is_a:
+        ref, size = ref.t(), size.t()
+    A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+    got = _gemm_dev(A, B, ta, tb, M, N, K).double()
+    assert ((got - ref).abs() <= K * 2.0 ** -24 * size + K * 2.0 ** -149).all()
 
 
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
