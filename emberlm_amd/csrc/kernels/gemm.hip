@@ -654,14 +654,29 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   const int rows_left = static_cast<int>(min(a.M - rw0, int64_t{BM}));
   const int cols_left = static_cast<int>(min(a.N - cw0, int64_t{BN}));
 
-  float bad = 0.f;  // NaN once some value is not finite
+  // Rows that are wanted (up to the 16-row group of a device-side count: the
+  // rest may come of memory that nobody filled).
+  const int64_t rows_end =
+      a.dyn && a.dyn_dim == 0 ? min((dyn_extent(a, a.M) + 15) / 16 * 16, a.M) : a.M;
+  const int rows_wanted = static_cast<int>(min(rows_end - rw0, int64_t{BM}));
+  // Whether a value that is wanted is not finite; ALL: every value is looked at.
+  const auto not_finite = [&](auto all) {
+    constexpr bool kAll = decltype(all)::value;
+    float bad = 0.f;  // NaN once some value is not finite
 #pragma unroll
-  for (int i = 0; i < FI; ++i)
+    for (int i = 0; i < FI; ++i)
 #pragma unroll
-    for (int j = 0; j < FJ; ++j)
+      for (int j = 0; j < FJ; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) bad = __builtin_fmaf(acc[i][j][e], 0.f, bad);
-  if (__builtin_expect(__any(bad != bad), 0)) {
+        for (int e = 0; e < 16; ++e) {
+          const bool wanted = kAll || (row_of(i, e) + lrow < rows_wanted && col_of(j) < cols_left);
+          bad = __builtin_fmaf(wanted ? acc[i][j][e] : 0.f, 0.f, bad);
+        }
+    return __any(bad != bad);
+  };
+  bool redo = not_finite(std::true_type{});
+  if (redo && (rows_wanted < BM / kWM || cols_left < BN / 2)) redo = not_finite(std::false_type{});
+  if (__builtin_expect(redo, 0)) {
     // This wave's tile in fp32 from global memory, 32x32 at a time.
     for (int t = 0; t < FI * FJ; ++t) {
       const int i = t / FJ, j = t % FJ;

@@ -862,6 +862,51 @@ def test_gemm_split_small_operands(ta, tb, small_is_a, M, N, K, t):
     assert ((got - ref).abs() <= K * 2.0 ** -24 * size + K * 2.0 ** -149).all()
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(140, 132, 52), (500, 124, 1000), (4092, 2052, 260),
+                                   (4092, 4092, 64)])
+def test_gemm_bits_do_not_depend_on_row_padding(ta, tb, M, N, K):
+    """What lies between the rows of either operand reaches no result, its bits included."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    ra, ca = (K, M) if ta else (M, K)
+    rb, cb = (N, K) if tb else (K, N)
+    need = capi.lib().ember_gemm_f32_workspace_bytes(M, N, K, 1)
+    ws = empty((max(need // 4, 1),))
+    A = torch.randn(ra, ca + 36, device="cuda", generator=g)
+    B = torch.randn(rb, cb + 36, device="cuda", generator=g)
+    got = []
+    for pad in (0.0, float("nan")):
+        A[:, ca:], B[:, cb:] = pad, pad
+        Cm = empty((M, N))
+        call("ember_gemm_f32_ws", ta, tb, M, N, K, 1.0, p(A), ca + 36, 0, p(B), cb + 36, 0, 0.0,
+             p(Cm), N, 0, 1, p(ws), need, None)
+        got.append(Cm)
+    assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("M,N,K,count", [(304, 260, 64, 131), (304, 260, 1024, 40),
+                                         (4096, 4096, 64, 1000)])
+@pytest.mark.parametrize("tb", [0, 1])
+def test_gemm_dyn_bits_do_not_depend_on_rows_past_the_count(M, N, K, count, tb):
+    """Rows past the count's 16-row group may hold anything (the LM head's stale rows)."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    A = torch.randn(M, K, device="cuda", generator=g)
+    B = torch.randn((N, K) if tb else (K, N), device="cuda", generator=g)
+    cnt = torch.tensor([count], device="cuda")
+    need = capi.lib().ember_gemm_f32_workspace_bytes(M, N, K, 1)
+    ws = empty((max(need // 4, 1),))
+    end = -(-count // 16) * 16
+    A[count:end] = 0.0
+    got = []
+    for stale in (1.0, float("nan")):
+        A[end:] = stale
+        Cm = empty((M, N))
+        call("ember_gemm_f32_dyn", 0, tb, M, N, K, 1.0, p(A), K, p(B), B.shape[1], 0.0, p(Cm), N,
+             p(cnt), 0, 0, p(ws), need, None)
+        got.append(Cm[:end])
+    assert torch.equal(*got) and not got[1][count:].any()
+
+
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
 def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
     """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
