@@ -480,7 +480,7 @@ struct SplitTile {
 // bias of sums that stay the same size along K or grow as sqrt(K), and all
 // but 9% where they grow as K (nothing here depends on a row's or column's
 // place).  K splits start negated by the parity of the number's count of ones
-// (0 1 1 0 1 0 0 1 ...).  Turning 256 accumulators costs about one stage.
+// (0 1 1 0 1 0 0 1 ...); the products of a batch all start alike.  Turning 256 accumulators costs about one stage.
 //
 // What the split cannot give: an infinity or NaN has no three parts, nor has a
 // value of 2^104 or more once scaled; such a result, or one past 2^80, is not
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   const int64_t nk = (K + 15) / 16;
   const int ra = g * TA::kHalf + (wm * (BM / kWM) + r) * 16;
   const int rb = TA::kBytes + g * TB::kHalf + (wn * (BN / 2) + r) * 16;
-  const bool start = __builtin_popcountll(bz) & 1;  // negated
+  const bool start = a.kchunk > 0 && (__builtin_popcountll(bz) & 1);  // negated
   if (nk > 0) {
     const int64_t pairs = (nk + 1) / 2;  // an odd nk's last stage is all zeros
     const int64_t turn[3] = {(pairs * 212) >> 10, (pairs * 724) >> 10, pairs};

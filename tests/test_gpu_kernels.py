@@ -907,6 +907,19 @@ def test_gemm_dyn_bits_do_not_depend_on_rows_past_the_count(M, N, K, count, tb):
     assert torch.equal(*got) and not got[1][count:].any()
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(60, 68, 36), (256, 260, 512)])
+def test_gemm_batch_place_does_not_change_bits(ta, tb, M, N, K):
+    """The same pair of matrices gives the same bits at every place of a batch."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    A = torch.randn((K, M) if ta else (M, K), device="cuda", generator=g).repeat(9, 1, 1)
+    B = torch.randn((N, K) if tb else (K, N), device="cuda", generator=g).repeat(9, 1, 1)
+    Cm = empty((9, M, N))
+    call("ember_gemm_f32", ta, tb, M, N, K, 1.0, p(A), A.shape[2], M * K, p(B), B.shape[2], N * K,
+         0.0, p(Cm), N, M * N, 9, None)
+    assert torch.equal(Cm, Cm[:1].expand_as(Cm))
+
+
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
 def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
     """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
