@@ -69,13 +69,13 @@ __device__ __forceinline__ int64_t dyn_extent(const GemmArgs& a, int64_t full) {
   return min(max(*a.dyn - a.dyn_base, int64_t{0}), full);
 }
 
-template <bool KC, int ROWS, int BK>
+template <bool KC, int ROWS, int BK, int THREADS>
 struct Stage {
   static constexpr int kStride = KC ? (BK + 4) : (ROWS + 8);
   static constexpr int kSize = KC ? ROWS * (BK + 4) : BK * (ROWS + 8);
   static constexpr int kChunks = ROWS * BK / 4;           // float4 chunks per tile
-  static constexpr int kPerThread = kChunks / kThreads;   // loads per thread
-  static_assert(kChunks % kThreads == 0, "tile not divisible among threads");
+  static constexpr int kPerThread = kChunks / THREADS;    // loads per thread
+  static_assert(kChunks % THREADS == 0, "tile not divisible among threads");
 
   f32x4 reg[kPerThread];
 
@@ -86,7 +86,7 @@ struct Stage {
                                        int64_t K, int64_t row0, int64_t k0) {
 #pragma unroll
     for (int p = 0; p < kPerThread; ++p) {
-      const int c = threadIdx.x + p * kThreads;
+      const int c = threadIdx.x + p * THREADS;
       int64_t r, k;
       if (KC) {
         r = row0 + c / (BK / 4);
@@ -125,7 +125,7 @@ struct Stage {
   __device__ __forceinline__ void store(float* __restrict__ lds) const {
 #pragma unroll
     for (int p = 0; p < kPerThread; ++p) {
-      const int c = threadIdx.x + p * kThreads;
+      const int c = threadIdx.x + p * THREADS;
       int off;
       if (KC) {
         off = (c / (BK / 4)) * kStride + 4 * (c % (BK / 4));
@@ -174,40 +174,31 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& a, int& tm, int& tn)
   tn = in / gsz;
 }
 
-template <bool A_KC, bool B_KC, bool VEC, int BM, int BN, int OCC>
-__global__ __launch_bounds__(kThreads, OCC) void gemm_f32_mfma(GemmArgs a) {
-  using SA = Stage<A_KC, BM, kBK>;
-  using SB = Stage<B_KC, BN, kBK>;
-  constexpr int FI = BM / 64, FJ = BN / 64;             // 32x32 tiles per wave
+// The LDS of one output tile on the fp32 MFMAs, and that tile (see the header):
+// rows m0 ..., columns n0 ... of C, over K.
+template <bool A_KC, bool B_KC, int BM, int BN, int THREADS>
+constexpr int kFp32LdsFloats =
+    2 * (Stage<A_KC, BM, kBK, THREADS>::kSize + Stage<B_KC, BN, kBK, THREADS>::kSize);
+
+template <bool A_KC, bool B_KC, bool VEC, int BM, int BN, int THREADS>
+__device__ __forceinline__ void fp32_tile(const GemmArgs& a, const float* __restrict__ A,
+                                          const float* __restrict__ B, float* __restrict__ C,
+                                          int64_t K, int64_t m0, int64_t n0, float* lds) {
+  using SA = Stage<A_KC, BM, kBK, THREADS>;
+  using SB = Stage<B_KC, BN, kBK, THREADS>;
+  constexpr int kWM = THREADS / 128;                    // waves along M; two along N
+  constexpr int FI = BM / (32 * kWM), FJ = BN / 64;     // 32x32 tiles per wave
   constexpr int NR = FI * (A_KC ? 1 : 4) + FJ * (B_KC ? 1 : 4);  // LDS reads per slab
   constexpr int NW = SA::kPerThread + SB::kPerThread;   // LDS stores per stage
   constexpr int NM = 4 * FI * FJ;                       // MFMAs per slab
-  __shared__ __attribute__((aligned(16))) float lds_a[2][SA::kSize];
-  __shared__ __attribute__((aligned(16))) float lds_b[2][SB::kSize];
-
-  int tm, tn;
-  tile_coords<BM, BN>(a, tm, tn);
-  const int64_t bz = blockIdx.y;
-  const float* __restrict__ A = a.A + bz * a.sA;
-  const float* __restrict__ B = a.B + bz * a.sB;
-  float* __restrict__ C = a.C + bz * a.sC;
-  int64_t K = a.kchunk > 0 ? min(a.kchunk, a.K - bz * a.kchunk) : a.K;
-  const int64_t m0 = static_cast<int64_t>(tm) * BM;
-  const int64_t n0 = static_cast<int64_t>(tn) * BN;
-  if (a.dyn) {  // uniform per block: the whole block leaves or none of it
-    if (a.dyn_dim == 0) {
-      if (m0 >= dyn_extent(a, a.M)) return;
-    } else {
-      K = min(K, (dyn_extent(a, K) + 15) / 16 * 16);
-      if (K == 0 && a.beta == 1.f && !a.D) return;  // C stays as it is
-    }
-  }
+  float* const lds_a[2] = {lds, lds + SA::kSize};
+  float* const lds_b[2] = {lds + 2 * SA::kSize, lds + 2 * SA::kSize + SB::kSize};
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int g = lane >> 5, r = lane & 31;
-  const int arow = wm * (BM / 2) + r, brow = wn * (BN / 2) + r;
+  const int arow = wm * (BM / kWM) + r, brow = wn * (BN / 2) + r;
 
   f32x16 acc[FI][FJ];
 #pragma unroll
@@ -295,7 +286,7 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_mfma(GemmArgs a) {
       if (col >= a.N) continue;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int64_t row = m0 + wm * (BM / 2) + i * 32 + 8 * (e >> 2) + 4 * g + (e & 3);
+        const int64_t row = m0 + wm * (BM / kWM) + i * 32 + 8 * (e >> 2) + 4 * g + (e & 3);
         if (row < a.M) {
           float* dst = C + row * a.ldc + col;
           const float v = a.alpha * acc[i][j][e];
@@ -305,6 +296,27 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_mfma(GemmArgs a) {
     }
 }
 
+template <bool A_KC, bool B_KC, bool VEC, int BM, int BN, int OCC>
+__global__ __launch_bounds__(kThreads, OCC) void gemm_f32_mfma(GemmArgs a) {
+  __shared__ __attribute__((aligned(16))) float lds[kFp32LdsFloats<A_KC, B_KC, BM, BN, kThreads>];
+
+  int tm, tn;
+  tile_coords<BM, BN>(a, tm, tn);
+  const int64_t bz = blockIdx.y;
+  int64_t K = a.kchunk > 0 ? min(a.kchunk, a.K - bz * a.kchunk) : a.K;
+  const int64_t m0 = static_cast<int64_t>(tm) * BM;
+  const int64_t n0 = static_cast<int64_t>(tn) * BN;
+  if (a.dyn) {  // uniform per block: the whole block leaves or none of it
+    if (a.dyn_dim == 0) {
+      if (m0 >= dyn_extent(a, a.M)) return;
+    } else {
+      K = min(K, (dyn_extent(a, K) + 15) / 16 * 16);
+      if (K == 0 && a.beta == 1.f && !a.D) return;  // C stays as it is
+    }
+  }
+  fp32_tile<A_KC, B_KC, VEC, BM, BN, kThreads>(a, a.A + bz * a.sA, a.B + bz * a.sB,
+                                               a.C + bz * a.sC, K, m0, n0, lds);
+}
 
 // ------------------------------------------------- bf16 matrix cores, fp32 in
 // Every fp32 value is the sum of three bf16 values exactly (8 + 8 + 8
@@ -499,6 +511,8 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   constexpr int FI = BM / (32 * kWM), FJ = BN / 64;      // 32x32 tiles per wave
   constexpr int kStage = TA::kBytes + TB::kBytes;
   __shared__ __attribute__((aligned(256))) char lds[2 * kStage];
+  __shared__ int redo_flag;  // some wanted value of the block's is not finite
+  if (threadIdx.x == 0) redo_flag = 0;
 
   int tm, tn;
   tile_coords<BM, BN>(a, tm, tn);
@@ -644,7 +658,7 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   // The lane's place in the output: register e of tile (i, j) is row slot
   // x = 8 (e / 4) + 4 g + e % 4 of MFMA tile i and column slot r of tile j.
   const int64_t rw0 = m0 + wm * (BM / kWM), cw0 = n0 + wn * (BN / 2);
-  if (rw0 >= a.M || cw0 >= a.N) return;
+  const bool mine = rw0 < a.M && cw0 < a.N;  // the wave has output
   const auto row_of = [&](int i, int e) {  // its uniform part; the lane's is lrow
     const int x = 8 * (e >> 2) + (e & 3);
     return A_KC || TA::P == 1 ? i * 32 + x : FI * x + i;
@@ -674,36 +688,29 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
         }
     return __any(bad != bad);
   };
-  bool redo = not_finite(std::true_type{});
-  if (redo && (rows_wanted < BM / kWM || cols_left < BN / 2)) redo = not_finite(std::false_type{});
-  if (__builtin_expect(redo, 0)) {
-    // This wave's tile in fp32 from global memory, 32x32 at a time.
-    for (int t = 0; t < FI * FJ; ++t) {
-      const int i = t / FJ, j = t % FJ;
-      const int64_t ar = min(rw0 + (A_KC || TA::P == 1 ? i * 32 + r : FI * r + i), a.M - 1);
-      const int64_t bc = min(cw0 + col_of(j), a.N - 1);
-      const float* pa = A_KC ? A + ar * a.lda : A + ar;
-      const float* pb = B_KC ? B + bc * a.ldb : B + bc;
-      const int64_t sa = A_KC ? 1 : a.lda, sb = B_KC ? 1 : a.ldb;
-      f32x16 v;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) v[e] = 0.f;
-      for (int64_t k = g; k < K + g; k += 2) {
-        const float x = k < K ? pa[k * sa] : 0.f, y = k < K ? pb[k * sb] : 0.f;
-        v = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, v, 0, 0, 0);
+  if (nk > 0) {
+    bool redo = mine && not_finite(std::true_type{});
+    if (redo && (rows_wanted < BM / kWM || cols_left < BN / 2))
+      redo = not_finite(std::false_type{});
+    if (redo && lane == 0) redo_flag = 1;
+    wait_lgkm0();
+    block_barrier();
+    if (__builtin_expect(redo_flag, 0)) {
+      // The block's tile on the fp32 MFMAs, 32x64 per wave at a time (64x64 would
+      // spill the registers of three blocks per CU).
+      constexpr int kM = 32 * kWM;
+      static_assert(kFp32LdsFloats<A_KC, B_KC, kM, 128, THREADS> * 4 <= 2 * kStage, "LDS");
+      for (int t = 0; t < (BM / kM) * (BN / 128); ++t) {
+        const int64_t m = m0 + kM * (t / (BN / 128)), n = n0 + 128 * (t % (BN / 128));
+        if (m >= a.M || n >= a.N) continue;
+        __syncthreads();  // the tile before has read its LDS
+        fp32_tile<A_KC, B_KC, true, kM, 128, THREADS>(a, A, B, C, K, m, n,
+                                                      reinterpret_cast<float*>(lds));
       }
-      if (col_of(j) >= cols_left) continue;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int64_t row = rw0 + row_of(i, e) + lrow, col = cw0 + col_of(j);
-        if (row >= a.M) continue;
-        float* dst = C + row * a.ldc + col;
-        const float x = a.alpha * v[e];
-        *dst = (a.beta != 0.f) ? x + a.beta * *addend(a, dst, row, col) : x;
-      }
+      return;
     }
-    return;
   }
+  if (!mine) return;
 
   const float back = start ? -kUnscale : kUnscale;
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -920,6 +920,52 @@ def test_gemm_batch_place_does_not_change_bits(ta, tb, M, N, K):
     assert torch.equal(Cm, Cm[:1].expand_as(Cm))
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(140, 132, 52), (300, 260, 1024), (4092, 2052, 260),
+                                   (8196, 2564, 96)])
+def test_gemm_add_with_a_nan_row_and_column(ta, tb, M, N, K):
+    """Tiles taken again in fp32, at each tile shape and with the addend: a NaN row and
+    column, the rest as fp32 sums of K terms."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.randn(n, K, device="cuda", generator=g) for n in (M, N))
+    D = torch.randn(M, N, device="cuda", generator=g)
+    ref = a.double() @ b.double().t().contiguous() + D
+    a[M // 2, 1] = b[N // 3, 0] = float("nan")
+    A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+    need = capi.lib().ember_gemm_f32_workspace_bytes(M, N, K, 1)
+    ws = empty((max(need // 4, 1),))
+    for Cm in (empty((M, N)), D):   # D separate, then D = C
+        call("ember_gemm_f32_add", ta, tb, M, N, K, 1.0, p(A), A.shape[1], p(B), B.shape[1], p(D), N,
+             p(Cm), N, p(ws), need, None)
+        bad = torch.isnan(Cm)
+        assert bad[M // 2].all() and bad[:, N // 3].all() and bad.sum().item() == M + N - 1
+        d = (Cm.double() - ref).masked_fill(bad, 0.0)
+        assert d.abs().max().item() <= 2e-6 * K ** 0.5 * max(1.0, ref.abs().max().item() / K ** 0.5)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0)])
+def test_gemm_time_with_nan_stays_near_that_of_fp32(ta, tb):
+    """A diverged run's products: all tiles taken again on the fp32 MFMAs, which are 2.7
+    times slower, on top of the first time (3.7 in all; 6 leaves room for staging)."""
+    M, N, K = 4096, 4096, 2048
+    B = torch.randn((N, K) if tb else (K, N), device="cuda")
+    best = []
+    for fill in (1.0, float("nan")):
+        A = torch.full((K, M) if ta else (M, K), fill, device="cuda").add_(
+            torch.randn((K, M) if ta else (M, K), device="cuda"))
+        times = []
+        for _ in range(6):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            Cm = _gemm_dev(A, B, ta, tb, M, N, K)
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1))
+        best.append(min(times))
+        assert torch.isnan(Cm).all() == (fill != fill)
+    assert best[1] <= 6 * best[0], best
+
+
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
 def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
     """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
