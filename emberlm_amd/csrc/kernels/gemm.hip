@@ -497,6 +497,12 @@ struct SplitTile {
 // What the split cannot give: an infinity or NaN has no three parts, nor has a
 // value of 2^104 or more once scaled; such a result, or one past 2^80, is not
 // finite, which is found here, and it is taken again in fp32.
+// The 512-thread tile has the registers for a second set of sums and adds up K
+// in segments of at most kSegK, an even number of them, with the same signs as
+// K splits: as exact as that many splits (1000x2048x2048 unsplit 4.85e-7 ->
+// 2.4e-7 in the 2-norm) without their planes.
+constexpr int kSegK = 256;
+
 // THREADS = 256: 4 waves in 2x2, wave tiles (BM/2)x(BN/2); 512: 8 waves in
 // 4x2.  LDS is double buffered.  A 256x256 block has a CU to itself and one wave per SIMD, so the
 // order of the wave's own instructions is what keeps the matrix core busy:
@@ -510,6 +516,8 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   constexpr int kWM = THREADS / 128;                     // waves along M; two along N
   constexpr int FI = BM / (32 * kWM), FJ = BN / 64;      // 32x32 tiles per wave
   constexpr int kStage = TA::kBytes + TB::kBytes;
+  constexpr bool kSegs = THREADS == 512;                 // K is summed in segments
+  constexpr int64_t kSegPairs = kSegK / 32;
   __shared__ __attribute__((aligned(256))) char lds[2 * kStage];
   __shared__ int redo_flag;  // some wanted value of the block's is not finite
   if (threadIdx.x == 0) redo_flag = 0;
@@ -552,9 +560,22 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   if (nk > 0) {
     const int64_t pairs = (nk + 1) / 2;  // an odd nk's last stage is all zeros
     const int64_t turn[3] = {(pairs * 212) >> 10, (pairs * 724) >> 10, pairs};
+    // kSegs: segments of `len` pairs, the first `more` of them one longer; one
+    // for a short K split, whose neighbours start with the other sign.
+    const unsigned segs =
+        pairs > (a.kchunk > 0 ? kSegPairs : 1)
+            ? 2 * static_cast<unsigned>((pairs + 2 * kSegPairs - 1) / (2 * kSegPairs))
+            : 1;
+    const unsigned len = static_cast<unsigned>(pairs) / segs;
+    const unsigned more = static_cast<unsigned>(pairs) - len * segs;
+    unsigned seg = 0;
+    int64_t seg_end = len + (more > 0);
+    const auto seg_neg = [&](unsigned i) { return start != ((__builtin_popcount(i) & 1) != 0); };
     float scale_b;  // of the values stored, which belong to pair `at`
     const auto sign_at = [&](int64_t at) {
-      scale_b = start != (at >= turn[0] && at < turn[1]) ? -kScale : kScale;
+      const bool neg = kSegs ? seg_neg(at < seg_end ? seg : seg + 1)
+                             : start != (at >= turn[0] && at < turn[1]);
+      scale_b = neg ? -kScale : kScale;
     };
     sign_at(0);
     TA ta;
@@ -639,18 +660,49 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
       }
     };
     int64_t p = 0;
-#pragma unroll
-    for (int part = 0; part < 3; ++part) {
-      while (p < turn[part]) {
+    const auto run_to = [&](int64_t end) {
+      while (p < end) {
         stage(std::integral_constant<int, 0>{});
         sign_at(++p);
         stage(std::integral_constant<int, 1>{});
       }
-      if (part < 2) {
+    };
+    if constexpr (kSegs) {
+      f32x16 sum[FI][FJ];
+#pragma unroll
+      for (int i = 0; i < FI; ++i)
+#pragma unroll
+        for (int j = 0; j < FJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sum[i][j][e] = 0.f;
+      for (; seg < segs; ++seg) {
+        run_to(seg_end);
+        seg_end += len + (seg + 1 < more);
+        const float sign = seg_neg(seg) ? -1.f : 1.f;
 #pragma unroll
         for (int i = 0; i < FI; ++i)
 #pragma unroll
-          for (int j = 0; j < FJ; ++j) acc[i][j] = -acc[i][j];
+          for (int j = 0; j < FJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              sum[i][j][e] = __builtin_fmaf(sign, acc[i][j][e], sum[i][j][e]);
+              acc[i][j][e] = 0.f;
+            }
+      }
+#pragma unroll
+      for (int i = 0; i < FI; ++i)
+#pragma unroll
+        for (int j = 0; j < FJ; ++j) acc[i][j] = sum[i][j];
+    } else {
+#pragma unroll
+      for (int part = 0; part < 3; ++part) {
+        run_to(turn[part]);
+        if (part < 2) {
+#pragma unroll
+          for (int i = 0; i < FI; ++i)
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) acc[i][j] = -acc[i][j];
+        }
       }
     }
   }
@@ -712,7 +764,7 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   }
   if (!mine) return;
 
-  const float back = start ? -kUnscale : kUnscale;
+  const float back = start && !kSegs ? -kUnscale : kUnscale;
 #if defined(__HIP_DEVICE_COMPILE__)
   // Stores (and the beta term's loads) through buffer resources based at this
   // wave's first output row of C (and of D): a row's byte offset splits into a
@@ -1034,16 +1086,24 @@ double predicted_us(const TileCost& t, int64_t M, int64_t N, int64_t K, int64_t 
 // From K = 4096 the split is all of `room`: shorter partial sums are also what
 // keeps the error of long ones down (a weight gradient's terms vary along the
 // tokens; 1024x2048x32768 in 8 chunks instead of 16 was 1.5 times further
-// from 64-bit sums, and 4% faster).
+// from 64-bit sums, and 4% faster).  Below that, a grid of few tiles is summed
+// in segments of at most kMaxChain from K = 512, which the 512-thread tile does
+// by itself and the others only by a split: 2048x1024x2048 unsplit was 1.66
+// times further from 64-bit sums than in eight fp32 chunks of 256.
+constexpr int64_t kMaxChain = 352;  // 0.85 sqrt(352 / 256) = 1.0 of such a chunk's error
+
 SplitPlan make_split_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t room,
                           int tiles) {
   SplitPlan best{1, 1, 0};
   double least = 1e30;
+  const bool short_chains =
+      room > 1 && K >= 512 && K < 4096 && 2 * cdiv(M, 128) * cdiv(N, 128) <= kCUs;
   for (int t = 0; t < tiles; ++t)
     for (int64_t s = K >= 4096 ? room : 1; s <= room; ++s) {
       const int64_t chunk = s > 1 ? cdiv(cdiv(K, s), 32) * 32 : K;
       const int64_t n = s > 1 ? cdiv(K, chunk) : 1;  // at most s
       if (t == 0 && cdiv(M, 128) * cdiv(N, 128) * batch * n > kCUs) continue;  // one round only
+      if (t > 0 && short_chains && chunk > kMaxChain) continue;
       double us = predicted_us(kTiles[t], M, N, chunk, batch, n);
       if (n > 1) us += 2.45 + static_cast<double>((n + 1) * M * N) * 4 / 5.21e6;
       if (us < least) {

@@ -966,6 +966,25 @@ def test_gemm_time_with_nan_stays_near_that_of_fp32(ta, tb):
     assert best[1] <= 6 * best[0], best
 
 
+@pytest.mark.parametrize("ta,tb,M,N,K", [
+    (1, 0, 2048, 1024, 2048), (0, 1, 1000, 2048, 2048), (0, 1, 968, 1024, 3072),
+    (0, 1, 27, 8192, 2048), (0, 0, 562, 2048, 1000), (1, 1, 2048, 1024, 4092),
+    (1, 0, 1024, 2048, 3605), (0, 1, 256, 576, 768),
+])
+def test_gemm_few_tiles_sum_k_in_short_chains(ta, tb, M, N, K):
+    """Products of few tiles with their workspace, K = 512 to 4095: no further from 64 bits
+    than fp32 sums of two k at a time in chunks of 256.  Those: 128 roundings of a sum that
+    grows with its square root, each 0.6 of 2^-24 (rms), 0.6 * 2^-24 * sqrt(128 / 2); 5%
+    for chunks that come out longer."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g)
+    A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+    ref = a.double() @ b.double().t().contiguous()
+    d = _gemm_dev(A, B, ta, tb, M, N, K).double() - ref
+    assert (d.norm() / ref.norm()).item() <= 1.05 * 0.6 * 2.0 ** -24 * 8
+    assert abs(d.mean().item()) <= 3e-8 * ref.abs().mean().item()
+
+
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
 def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
     """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
