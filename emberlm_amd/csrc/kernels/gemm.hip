@@ -191,8 +191,8 @@ __device__ __forceinline__ void fp32_tile(const GemmArgs& a, const float* __rest
   constexpr int NR = FI * (A_KC ? 1 : 4) + FJ * (B_KC ? 1 : 4);  // LDS reads per slab
   constexpr int NW = SA::kPerThread + SB::kPerThread;   // LDS stores per stage
   constexpr int NM = 4 * FI * FJ;                       // MFMAs per slab
-  float* const lds_a[2] = {lds, lds + SA::kSize};
-  float* const lds_b[2] = {lds + 2 * SA::kSize, lds + 2 * SA::kSize + SB::kSize};
+  float* const lds_a = lds;                  // two stages each
+  float* const lds_b = lds + 2 * SA::kSize;
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -214,16 +214,16 @@ __device__ __forceinline__ void fp32_tile(const GemmArgs& a, const float* __rest
   if (nk > 0) {
     sa.template load<VEC>(A, a.lda, a.M, K, m0, 0);
     sb.template load<VEC>(B, a.ldb, a.N, K, n0, 0);
-    sa.store(lds_a[0]);
-    sb.store(lds_b[0]);
+    sa.store(lds_a);
+    sb.store(lds_b);
   }
   __syncthreads();
 
   f32x4 fa0[FI], fb0[FJ], fa1[FI], fb1[FJ];
 #pragma unroll
-  for (int i = 0; i < FI; ++i) fa0[i] = SA::frag(lds_a[0], arow + i * 32, 0, g);
+  for (int i = 0; i < FI; ++i) fa0[i] = SA::frag(lds_a, arow + i * 32, 0, g);
 #pragma unroll
-  for (int j = 0; j < FJ; ++j) fb0[j] = SB::frag(lds_b[0], brow + j * 32, 0, g);
+  for (int j = 0; j < FJ; ++j) fb0[j] = SB::frag(lds_b, brow + j * 32, 0, g);
 
   for (int64_t kt = 0; kt < nk; ++kt) {
     const int cur = static_cast<int>(kt & 1);
@@ -232,10 +232,10 @@ __device__ __forceinline__ void fp32_tile(const GemmArgs& a, const float* __rest
     const int64_t knext = (kt + 1 < nk ? kt + 1 : kt) * kBK;
     sa.template load<VEC>(A, a.lda, a.M, K, m0, knext);
     sb.template load<VEC>(B, a.ldb, a.N, K, n0, knext);
-    const float* la = lds_a[cur];
-    const float* lb = lds_b[cur];
-    float* na = lds_a[cur ^ 1];
-    float* nb = lds_b[cur ^ 1];
+    const float* la = lds_a + cur * SA::kSize;
+    const float* lb = lds_b + cur * SB::kSize;
+    float* na = lds_a + (cur ^ 1) * SA::kSize;
+    float* nb = lds_b + (cur ^ 1) * SB::kSize;
 
 #pragma unroll
     for (int i = 0; i < FI; ++i) fa1[i] = SA::frag(la, arow + i * 32, 1, g);
@@ -1165,13 +1165,16 @@ int launch_split(const GemmArgs& a, int tile, bool a_kc, bool b_kc, int64_t ny, 
                      : launch_split_tile<256, 256, 256, 1>(a, a_kc, b_kc, ny, st);
 }
 
-// How many of kTiles gemm_f32_split can use for these operands: none unless
-// their rows are float4 rows that end on a whole float4; else those for which
+// How many of kTiles gemm_f32_split can use for these operands: none for a K of
+// at most 8, where the fp32 MFMAs, which round a lone product to nearest, are
+// closer to 64 bits when some terms are zero (K = 4 with one term: 2.5e-8
+// against 3.4e-8 in the 2-norm; from K = 12 with three terms on, further) and
+// the stores of C are what takes the time; none unless their rows are float4 rows that end on a whole float4; else those for which
 // every byte offset inside a block's operand stage and output tile (the
 // tile's rows of a K-contiguous operand and of C, 16 k of the other) stays
 // below 2^31.
 int split_tiles(const GemmArgs& a, bool a_kc, bool b_kc, bool vec) {
-  if (!vec || (a_kc ? a.K : a.M) % 4 != 0 || (b_kc ? a.K : a.N) % 4 != 0) return 0;
+  if (a.K <= 8 || !vec || (a_kc ? a.K : a.M) % 4 != 0 || (b_kc ? a.K : a.N) % 4 != 0) return 0;
   const auto fits = [&](int64_t rows) {
     const int64_t top = (int64_t{1} << 29) - 1024;  // floats
     return (a_kc ? rows - 1 : 16) * a.lda < top && (b_kc ? rows - 1 : 16) * a.ldb < top &&

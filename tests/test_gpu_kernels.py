@@ -985,6 +985,17 @@ def test_gemm_few_tiles_sum_k_in_short_chains(ta, tb, M, N, K):
     assert abs(d.mean().item()) <= 3e-8 * ref.abs().mean().item()
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(64, 512, 4), (140, 132, 8), (4096, 2048, 8)])
+def test_gemm_lone_products_of_a_short_k_round_to_nearest(ta, tb, M, N, K):
+    """K <= 8 with one term that is not zero: the fp32 product, bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b = torch.zeros(M, K, device="cuda"), torch.randn(N, K, device="cuda", generator=g)
+    a[:, K - 3] = torch.randn(M, device="cuda", generator=g)
+    A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+    assert torch.equal(_gemm_dev(A, B, ta, tb, M, N, K), a[:, K - 3, None] * b[None, :, K - 3])
+
+
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
 def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
     """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
