@@ -740,29 +740,18 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
         }
     return __any(bad != bad);
   };
-  if (nk > 0) {
-    bool redo = mine && not_finite(std::true_type{});
-    if (redo && (rows_wanted < BM / kWM || cols_left < BN / 2))
-      redo = not_finite(std::false_type{});
+  bool redo = nk > 0 && mine && not_finite(std::true_type{});
+  if (redo && (rows_wanted < BM / kWM || cols_left < BN / 2)) redo = not_finite(std::false_type{});
+  // Whether any wave of the block has to.  C is needed as it was only where the
+  // beta term may read it, so elsewhere the waves ask after their stores.
+  const auto block_redo = [&]() {
     if (redo && lane == 0) redo_flag = 1;
     wait_lgkm0();
     block_barrier();
-    if (__builtin_expect(redo_flag, 0)) {
-      // The block's tile on the fp32 MFMAs, 32x64 per wave at a time (64x64 would
-      // spill the registers of three blocks per CU).
-      constexpr int kM = 32 * kWM;
-      static_assert(kFp32LdsFloats<A_KC, B_KC, kM, 128, THREADS> * 4 <= 2 * kStage, "LDS");
-      for (int t = 0; t < (BM / kM) * (BN / 128); ++t) {
-        const int64_t m = m0 + kM * (t / (BN / 128)), n = n0 + 128 * (t % (BN / 128));
-        if (m >= a.M || n >= a.N) continue;
-        __syncthreads();  // the tile before has read its LDS
-        fp32_tile<A_KC, B_KC, true, kM, 128, THREADS>(a, A, B, C, K, m, n,
-                                                      reinterpret_cast<float*>(lds));
-      }
-      return;
-    }
-  }
-  if (!mine) return;
+    return redo_flag != 0;
+  };
+  const bool ask_first = a.beta != 0.f;
+  bool again = nk > 0 && ask_first && block_redo();
 
   const float back = start && !kSegs ? -kUnscale : kUnscale;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -776,46 +765,82 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(Dm + rw0 * ldd + cw0), 0, 0x7fffffff, 0x00020000);
   const int lc = static_cast<int>(lrow * a.ldc * 4), ld = static_cast<int>(lrow * ldd * 4);
-  // CHECKED: the wave tile reaches M.  BETA: the beta term is read, all 16
-  // values of an MFMA tile before the first is used (one wait per tile).
+  // CHECKED: the wave tile reaches M.  BETA: the beta term is read, 16 values
+  // before the first is used.  Where a lane has its FJ columns side by side (N
+  // is then whole float4s) they go in one access: 4 bytes at a time, 16 apart,
+  // were what a short K took its time for (8192x6144x32 TN 76 us).
+  constexpr int V = B_KC || TB::P == 1 ? 1 : FJ;
+  using Out = std::conditional_t<V == 4, u32x4, std::conditional_t<V == 2, u32x2, unsigned>>;
+  static_assert(V == 1 || V == TB::P, "a lane's columns");
   auto store_all = [&](auto checked, auto with_beta) {
     constexpr bool kChecked = decltype(checked)::value, kBeta = decltype(with_beta)::value;
 #pragma unroll
-    for (int j = 0; j < FJ; ++j) {
+    for (int j = 0; j < FJ; j += V) {
       const int col = col_of(j);
       if (col >= cols_left) continue;
 #pragma unroll
-      for (int i = 0; i < FI; ++i) {
-        float d[16];
+      for (int i = 0; i < FI; ++i)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int ru = row_of(i, e);
-          d[e] = 0.f;
-          if (kBeta && !(kChecked && ru + lrow >= rows_left))
-            d[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                 rd, ld + 4 * col, static_cast<int>(ru * ldd * 4), 0));
-        }
+        for (int e0 = 0; e0 < 16; e0 += 16 / V) {
+          float d[16 / V][V];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int ru = row_of(i, e);
-          if (kChecked && ru + lrow >= rows_left) continue;
-          const float v = a.alpha * __builtin_fmaf(back, acc[i][j][e], 0.f);  // +0 for a zero
-          const float out = kBeta ? v + a.beta * d[e] : v;
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, out), rc, lc + 4 * col,
-                                                static_cast<int>(ru * a.ldc * 4), 0);
+          for (int e = 0; e < 16 / V; ++e) {
+            const int ru = row_of(i, e0 + e);
+            Out x{};
+            if (kBeta && !(kChecked && ru + lrow >= rows_left)) {
+              const int at = ld + 4 * col, row = static_cast<int>(ru * ldd * 4);
+              if constexpr (V == 4) x = __builtin_amdgcn_raw_buffer_load_b128(rd, at, row, 0);
+              else if constexpr (V == 2) x = __builtin_amdgcn_raw_buffer_load_b64(rd, at, row, 0);
+              else x = __builtin_amdgcn_raw_buffer_load_b32(rd, at, row, 0);
+            }
+            __builtin_memcpy(d[e], &x, sizeof x);
+          }
+#pragma unroll
+          for (int e = 0; e < 16 / V; ++e) {
+            const int ru = row_of(i, e0 + e);
+            if (kChecked && ru + lrow >= rows_left) continue;
+            float out[V];
+#pragma unroll
+            for (int c = 0; c < V; ++c) {
+              const float v = a.alpha * __builtin_fmaf(back, acc[i][j + c][e0 + e], 0.f);  // +0 for a zero
+              out[c] = kBeta ? v + a.beta * d[e][c] : v;
+            }
+            Out x;
+            __builtin_memcpy(&x, out, sizeof x);
+            const int at = lc + 4 * col, row = static_cast<int>(ru * a.ldc * 4);
+            if constexpr (V == 4) __builtin_amdgcn_raw_buffer_store_b128(x, rc, at, row, 0);
+            else if constexpr (V == 2) __builtin_amdgcn_raw_buffer_store_b64(x, rc, at, row, 0);
+            else __builtin_amdgcn_raw_buffer_store_b32(x, rc, at, row, 0);
+          }
         }
-      }
     }
   };
   const bool full = rows_left >= BM / kWM;
-  if (a.beta != 0.f) {
-    if (full) store_all(std::false_type{}, std::true_type{});
-    else store_all(std::true_type{}, std::true_type{});
-  } else {
-    if (full) store_all(std::false_type{}, std::false_type{});
-    else store_all(std::true_type{}, std::false_type{});
+  if (mine && !again) {
+    if (a.beta != 0.f) {
+      if (full) store_all(std::false_type{}, std::true_type{});
+      else store_all(std::true_type{}, std::true_type{});
+    } else {
+      if (full) store_all(std::false_type{}, std::false_type{});
+      else store_all(std::true_type{}, std::false_type{});
+    }
   }
 #endif
+  if (nk > 0 && !ask_first) again = block_redo();
+  if (__builtin_expect(again, 0)) {
+    // The block's tile on the fp32 MFMAs, 32x64 per wave at a time (64x64 would
+    // spill the registers of three blocks per CU).
+    constexpr int kM = 32 * kWM;
+    static_assert(kFp32LdsFloats<A_KC, B_KC, kM, 128, THREADS> * 4 <= 2 * kStage, "LDS");
+    wait_vm_lgkm0<0>();  // this wave's stores are done before others write there
+    for (int t = 0; t < (BM / kM) * (BN / 128); ++t) {
+      const int64_t m = m0 + kM * (t / (BN / 128)), n = n0 + 128 * (t % (BN / 128));
+      if (m >= a.M || n >= a.N) continue;
+      __syncthreads();  // the tile before has read its LDS
+      fp32_tile<A_KC, B_KC, true, kM, 128, THREADS>(a, A, B, C, K, m, n,
+                                                    reinterpret_cast<float*>(lds));
+    }
+  }
 }
 
 // C = alpha * sum_{s<S} P[s] + beta * D (D = C when null), the split partials

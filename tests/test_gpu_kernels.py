@@ -996,6 +996,32 @@ def test_gemm_lone_products_of_a_short_k_round_to_nearest(ta, tb, M, N, K):
     assert torch.equal(_gemm_dev(A, B, ta, tb, M, N, K), a[:, K - 3, None] * b[None, :, K - 3])
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+def test_gemm_short_k_time_is_near_that_of_writing_c(ta, tb):
+    """K = 32 (a weight gradient of 32 tokens): the stores of C bound it.  Writing the same
+    200 MB by ember_fill (26 us) is the measure: 1.7 times that in row-long accesses, 3
+    when a lane stored four bytes at a time, 16 apart."""
+    M, N, K = 8192, 6144, 32
+    A = torch.randn((K, M) if ta else (M, K), device="cuda")
+    B = torch.randn((N, K) if tb else (K, N), device="cuda")
+    Cm = empty((M, N))
+    best = []
+    for run in (lambda: capi.call("ember_fill", p(Cm), M * N, 0.0, None),
+                lambda: capi.call("ember_gemm_f32", ta, tb, M, N, K, 1.0, p(A), A.shape[1], 0, p(B),
+                                  B.shape[1], 0, 0.0, p(Cm), N, 0, 1, None)):
+        times = []
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(10):
+                run()
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1))
+        best.append(min(times))
+    assert best[1] <= 2.3 * best[0], best
+
+
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
 def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
     """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
