@@ -368,7 +368,7 @@ struct SplitTile {
   static constexpr int kBytes = 3 * kPlane;
   const char* base;      // the tile's first element at the current stage
   int64_t left;          // bytes from there to the operand's end
-  int64_t step;          // bytes between stages
+  int64_t step;          // bytes of a k
   int voff;              // this lane's first element, bytes from base
   int soff[KC ? P : 4];  // uniform offsets of the lane's loads
   int woff;              // where the lane's first four k go in LDS
@@ -377,10 +377,10 @@ struct SplitTile {
 
   __device__ __forceinline__ void init(const float* X, int64_t ld, int64_t R, int64_t K,
                                        int64_t row0, int wave, int lane) {
+    step = KC ? 4 : 4 * ld;
     if constexpr (KC) {
       base = reinterpret_cast<const char*>(X + row0 * ld);
       left = ((R - row0 - 1) * ld + K) * 4;
-      step = 64;
       const int row = 16 * wave + (lane >> 2), quad = lane & 3;
       voff = static_cast<int>(row * ld * 4) + 16 * quad;
 #pragma unroll
@@ -389,7 +389,6 @@ struct SplitTile {
     } else {
       base = reinterpret_cast<const char*>(X + row0);
       left = ((K - 1) * ld + R - row0) * 4;
-      step = 64 * ld;
       const int quad = wave & 3, first = 64 * P * (wave >> 2);  // first row of the wave's
       voff = 4 * (first + P * lane);
 #pragma unroll
@@ -400,8 +399,7 @@ struct SplitTile {
 
   static constexpr int kLoads = KC ? P : 4;
   // Load q of the current stage.  Past the operand's end the buffer resource
-  // returns zeros, so no row or k is tested, except k past K in a
-  // K-contiguous row (`at`).
+  // returns zeros, so no row or k is tested.
   __device__ __forceinline__ void load(int q) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -416,14 +414,19 @@ struct SplitTile {
       reg[q] = __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0));
 #endif
   }
-  __device__ __forceinline__ void next() {
-    base += step;
-    left -= step;
-  }
-  __device__ __forceinline__ void load_all() {
+  // All loads of the current stage, of which `k` (four at a time) count.
+  __device__ __forceinline__ void load_all(int k = 16) {
 #pragma unroll
     for (int q = 0; q < kLoads; ++q) load(q);
-    next();
+    base += k * step;
+    left -= k * step;
+  }
+  // Zeros for the k of the loaded stage that don't.
+  __device__ __forceinline__ void mask(int k, int wave, int lane) {
+    if (k <= 4 * (KC ? lane & 3 : wave & 3)) {
+#pragma unroll
+      for (int q = 0; q < kLoads; ++q) reg[q] = Vec{};
+    }
   }
   // Element (k j of the lane's quad, row i of the lane's P).
   __device__ __forceinline__ float at(int j, int i) const {
@@ -433,17 +436,13 @@ struct SplitTile {
   }
   // The split of row i's four k, in kSteps steps of at most four VALU
   // operations for the spaces between MFMAs; the last stores the parts.
-  // MASK: a K-contiguous lane's k count only when `valid`.  `scale`: +-kScale.
+  // `scale`: +-kScale.
   static constexpr int kSteps = 7;
-  template <bool MASK>
-  __device__ __forceinline__ void split_step(SplitWork& w, int i, int step, char* lds, bool valid,
+  __device__ __forceinline__ void split_step(SplitWork& w, int i, int step, char* lds,
                                              float scale) const {
     if (step == 0) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float v = MASK && KC && !valid ? 0.f : at(j, i);
-        w.x[j] = v * scale;
-      }
+      for (int j = 0; j < 4; ++j) w.x[j] = at(j, i) * scale;
     } else if (step == 1 || step == 3) {
       const int p = step / 3;
       w.part[p] = u32x2{pack_bf16(w.x[0], w.x[1]), pack_bf16(w.x[2], w.x[3])};
@@ -460,13 +459,12 @@ struct SplitTile {
         *reinterpret_cast<u32x2*>(lds + woff + p * kPlane + i * (KC ? THREADS / 4 : 32) * 16) = w.part[p];
     }
   }
-  template <bool MASK>
-  __device__ __forceinline__ void store_all(char* lds, bool valid, float scale) const {
+  __device__ __forceinline__ void store_all(char* lds, float scale) const {
 #pragma unroll
     for (int i = 0; i < P; ++i) {
       SplitWork w;
 #pragma unroll
-      for (int t = 0; t < kSteps; ++t) split_step<MASK>(w, i, t, lds, valid, scale);
+      for (int t = 0; t < kSteps; ++t) split_step(w, i, t, lds, scale);
     }
   }
   // Part p of 32-slot tile t (from the wave's first), for lane offset `off`.
@@ -509,7 +507,7 @@ constexpr int kSegK = 256;
 // it is written out MFMA by MFMA and pinned (sched_barrier), two to eight
 // VALU operations of the split between two MFMAs of 32 cycles each.  Left to
 // the compiler, the same work ran at 207 TFLOP/s instead of 241.
-template <bool A_KC, bool B_KC, int BM, int BN, int THREADS, int OCC, bool TAIL>
+template <bool A_KC, bool B_KC, int BM, int BN, int THREADS, int OCC>
 __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   using TA = SplitTile<A_KC, BM, THREADS>;
   using TB = SplitTile<B_KC, BN, THREADS>;
@@ -558,7 +556,7 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   const int rb = TA::kBytes + g * TB::kHalf + (wn * (BN / 2) + r) * 16;
   const bool start = a.kchunk > 0 && (__builtin_popcountll(bz) & 1);  // negated
   if (nk > 0) {
-    const int64_t pairs = (nk + 1) / 2;  // an odd nk's last stage is all zeros
+    const int64_t pairs = (nk + 1) / 2;
     const int64_t turn[3] = {(pairs * 212) >> 10, (pairs * 724) >> 10, pairs};
     // kSegs: segments of `len` pairs, the first `more` of them one longer; one
     // for a short K split, whose neighbours start with the other sign.
@@ -582,13 +580,27 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
     TB tb;
     ta.init(A, a.lda, a.M, K, m0, wave, lane);
     tb.init(B, a.ldb, a.N, K, n0, wave, lane);
-    int64_t klane = K - 4 * (lane & 3);  // TAIL: k left from this lane's quad on
-    ta.load_all();
-    tb.load_all();
-    ta.template store_all<TAIL>(lds, klane > 0, kScale);
-    tb.template store_all<TAIL>(lds + TA::kBytes, klane > 0, scale_b);
-    ta.load_all();
-    tb.load_all();
+    // A K that is not whole pairs of stages begins with what is missing, an
+    // empty stage, a short one or both (a K-contiguous operand's K is whole
+    // float4s), so that the loop has no k to leave out.  Where neither operand
+    // is K-contiguous both end where memory says.
+    const int rest = static_cast<int>(K - 16 * (nk - 1));
+    const int first = !(A_KC || B_KC) ? 16 : nk & 1 ? 0 : rest;
+    const int second = !(A_KC || B_KC) || !(nk & 1) ? 16 : rest;
+    ta.load_all(first);
+    tb.load_all(first);
+    if (first < 16) {
+      ta.mask(first, wave, lane);
+      tb.mask(first, wave, lane);
+    }
+    ta.store_all(lds, kScale);
+    tb.store_all(lds + TA::kBytes, scale_b);
+    ta.load_all(second);
+    tb.load_all(second);
+    if (second < 16) {
+      ta.mask(second, wave, lane);
+      tb.mask(second, wave, lane);
+    }
     wait_lgkm0();
     block_barrier();
     bf16x8 fa[2][3], fb[2][FJ][3];
@@ -615,7 +627,6 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
       constexpr int kWork = kQuads * TA::kSteps;
       const char* cur = lds + kOdd * kStage;
       char* nxt = lds + (1 - kOdd) * kStage;
-      if (TAIL) klane -= 16;
       SplitWork w;
 #pragma unroll
       for (int i = 0; i < FI; ++i) {
@@ -647,10 +658,9 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
               for (int s = m * kWork / kSlots; s < (m + 1) * kWork / kSlots; ++s) {
                 const int q = s / TA::kSteps, st = s % TA::kSteps;
                 if (q < TA::P)
-                  ta.template split_step<TAIL>(w, q, st, nxt, klane > 0, kScale);
+                  ta.split_step(w, q, st, nxt, kScale);
                 else
-                  tb.template split_step<TAIL>(w, q - TA::P, st, nxt + TA::kBytes, klane > 0,
-                                               scale_b);
+                  tb.split_step(w, q - TA::P, st, nxt + TA::kBytes, scale_b);
                 if (s == TA::P * TA::kSteps - 1) ta.load_all();
                 if (s == kWork - 1) tb.load_all();
               }
@@ -1164,14 +1174,7 @@ int launch_split_t(GemmArgs a, int64_t ny, hipStream_t st) {
   a.tiles_m = static_cast<int>(cdiv(a.M, BM));
   a.tiles_n = static_cast<int>(cdiv(a.N, BN));
   dim3 grid(static_cast<unsigned>(a.tiles_m) * a.tiles_n, static_cast<unsigned>(ny));
-  // Stages run in pairs: a K-contiguous operand has to be masked past K unless
-  // every split is whole pairs (an MN-contiguous one ends where memory says).
-  const bool whole = (a.kchunk > 0 ? a.kchunk : a.K) % 32 == 0 && a.K % 32 == 0 &&
-                     !(a.dyn && a.dyn_dim == 1);
-  if ((A_KC || B_KC) && !whole)
-    gemm_f32_split<A_KC, B_KC, BM, BN, THREADS, OCC, true><<<grid, THREADS, 0, st>>>(a);
-  else
-    gemm_f32_split<A_KC, B_KC, BM, BN, THREADS, OCC, false><<<grid, THREADS, 0, st>>>(a);
+  gemm_f32_split<A_KC, B_KC, BM, BN, THREADS, OCC><<<grid, THREADS, 0, st>>>(a);
   return launch_status();
 }
 

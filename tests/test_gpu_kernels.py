@@ -1022,6 +1022,28 @@ def test_gemm_short_k_time_is_near_that_of_writing_c(ta, tb):
     assert best[1] <= 2.3 * best[0], best
 
 
+@pytest.mark.parametrize("tb", [0, 1])
+def test_gemm_ragged_k_takes_no_longer_than_the_next_whole_one(tb):
+    """K = 48 is not whole pairs of stages, K = 64 is (a tenth for the clock)."""
+    M, N = 8192, 6144
+    A, B = torch.randn(64 * M, device="cuda"), torch.randn(64 * N, device="cuda")
+    Cm = empty((M, N))
+    best = []
+    for K in (48, 64):
+        times = []
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(10):
+                capi.call("ember_gemm_f32", 0, tb, M, N, K, 1.0, p(A), K, 0, p(B), K if tb else N, 0,
+                          0.0, p(Cm), N, 0, 1, None)
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1))
+        best.append(min(times))
+    assert best[0] <= 1.1 * best[1], best
+
+
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
 def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
     """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
