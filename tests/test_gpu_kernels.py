@@ -714,32 +714,52 @@ def test_gemm_add_bitwise_equals_product_then_add(ta, tb, M, N, K):
         assert_close(host(Cm), O.matmul(a, b, ta, tb) + d, name="gemm add")
 
 
-@pytest.mark.parametrize("ta,tb,big", [(0, 1, "a"), (1, 0, "a"), (0, 0, "b"), (1, 1, "b")])
-def test_gemm_global_address_dma_bitwise_equals_buffer_dma(ta, tb, big):
-    """The DMA kernels copy operands into LDS through a buffer resource with
-    32-bit offsets unless some offset of the product reaches 2^31 bytes; then
-    with 64-bit global addresses.  A leading dimension large enough to force
-    the second form (a few strided rows of a 0.3-2.1 GB buffer) gives the same
-    bits as the compact operands, which take the first."""
-    M, N, K = 20, 20, 32
-    r = rng(11 + 2 * ta + tb)
+# The split kernel takes an operand whose block-tile rows (128 of a K-contiguous one, 16 k of
+# an M- or N-contiguous one) lie within (2^29 - 1024) floats; past that the fp32 kernel does.
+KC_LD, MN_LD = 4227320, 33554364     # the largest multiples of 4 that are within
+
+
+@pytest.mark.parametrize("ta,tb,big,K", [(0, 1, "a", 1024), (0, 1, "b", 36), (0, 0, "a", 36),
+                                         (1, 1, "b", 1024), (1, 0, "a", 32), (0, 0, "b", 32)])
+@pytest.mark.parametrize("over", [False, True])
+def test_gemm_rows_far_apart_just_under_and_over_the_split_limit(ta, tb, big, K, over):
+    """Under the limit: the bits of compact operands.  Over it: those of compact operands that
+    the fp32 kernel takes because their rows are not whole float4s.  The two differ, so each
+    side reaches its kernel; with a K split, and with a separate addend."""
+    M, N = 132, 140
+    r = rng(11 + 2 * ta + tb + K)
     a = r.standard_normal((K, M) if ta else (M, K)).astype(np.float32)
-    b = r.standard_normal((N, K) if tb else (K, N)).astype(np.float32)
-    want = gemm(a, b, ta, tb)
+    b = r.standard_normal((K, N) if not tb else (N, K)).astype(np.float32)
+    D = dev(r.standard_normal((M, N)).astype(np.float32))
     x = a if big == "a" else b
     rows, cols = x.shape
-    kc = (big == "a" and not ta) or (big == "b" and tb)
-    ld = (1 << 22) if kc else (1 << 24)   # 128 * ld or K * ld floats: 2^31 bytes
+    ld = (KC_LD if cols == K else MN_LD) + 4 * over
     X = torch.zeros((rows - 1) * ld + cols, device="cuda")
-    for i in range(rows):
-        X[i * ld: i * ld + cols].copy_(torch.from_numpy(x[i]))
-    Y = dev(b if big == "a" else a)
-    A, lda = (X, ld) if big == "a" else (Y, a.shape[1])
-    B, ldb = (X, ld) if big == "b" else (Y, b.shape[1])
-    Cm = empty((M, N))
-    call("ember_gemm_f32", int(ta), int(tb), M, N, K, 1.0, p(A), lda, 0, p(B), ldb, 0, 0.0,
-         p(Cm), N, 0, 1, None)
-    assert np.array_equal(host(Cm), want)
+    X.as_strided((rows, cols), (ld, 1)).copy_(torch.from_numpy(x))
+    need = capi.lib().ember_gemm_f32_workspace_bytes(M, N, K, 1)
+    assert (need > 0) == (K >= 512)
+    ws = empty((max(need // 4, 1),))
+
+    def run(name, X, ld):
+        Y = dev(b if big == "a" else a)
+        A, lda, B, ldb = (X, ld, Y, b.shape[1]) if big == "a" else (Y, a.shape[1], X, ld)
+        Cm = empty((M, N))
+        if name == "ws":
+            call("ember_gemm_f32_ws", ta, tb, M, N, K, 1.0, p(A), lda, 0, p(B), ldb, 0, 0.0, p(Cm),
+                 N, 0, 1, p(ws), need, None)
+        else:
+            call("ember_gemm_f32_add", ta, tb, M, N, K, 1.0, p(A), lda, p(B), ldb, p(D), N, p(Cm),
+                 N, p(ws), need, None)
+        return Cm
+
+    for name in ("ws", "add"):
+        got = run(name, X, ld)
+        whole = run(name, dev(x), cols)
+        odd = run(name, dev(np.pad(x, ((0, 0), (0, 1)))), cols + 1)
+        assert not torch.equal(whole, odd)
+        assert torch.equal(got, odd if over else whole)
+        want = O.matmul(a, b, bool(ta), bool(tb)) + (host(D) if name == "add" else 0.0)
+        assert_close(host(got), want, name="gemm " + name)
     del X
     torch.cuda.empty_cache()
 
@@ -780,16 +800,19 @@ def test_gemm_split_tile_edges_vs_float64(ta, tb, M, N, K):
 
 @pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
 def test_gemm_split_small_terms_and_exact_products(ta, tb):
-    """All 24 bits of both operands count (K = 4 with one nonzero term is exact), and
-    a sum of like-signed products gathers no bias over columns."""
-    M, N = 64, 512
+    """All 24 bits of either operand count (one nonzero term of K = 16, times a factor of few
+    bits, is the rounded product), and a sum of products gathers no bias."""
+    M, N, K = 64, 512, 16
     g = torch.Generator(device="cuda").manual_seed(5)
-    x = torch.randn(M, 1, device="cuda", generator=g)
-    a = torch.cat([x, torch.zeros(M, 3, device="cuda")], 1)
-    b = torch.ones(N, 4, device="cuda") * 3.0
-    A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
-    got = _gemm_dev(A, B, ta, tb, M, N, 4)
-    assert torch.equal(got, (3.0 * x).expand(M, N))
+    for m, n in ((M, N), (N, M)):   # the random factor in A, then in B
+        x = torch.randn(m, 1, device="cuda", generator=g)
+        a = torch.cat([x, torch.zeros(m, K - 1, device="cuda")], 1)
+        b = torch.full((n, K), 3.0, device="cuda")
+        if m == N:
+            a, b = b, a
+        A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+        got = _gemm_dev(A, B, ta, tb, M, N, K)
+        assert torch.equal(got if m == M else got.t(), (3.0 * x).expand(m, n))
     K = 4096
     a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g)
     A, B = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
