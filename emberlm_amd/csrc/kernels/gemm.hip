@@ -10,7 +10,8 @@
 // 0.157.  Against 64-bit sums its error is 0.85 of theirs (see the kernel).
 //
 // Fallback, gemm_f32_mfma (rows that are not whole aligned float4s, offsets
-// past 2 GB): v_mfma_f32_32x32x2_f32, tiles 128x128 (three blocks per CU) or
+// past 2 GB, K of at most 8), whose tile also serves the split kernel's results
+// that are not finite: v_mfma_f32_32x32x2_f32, tiles 128x128 (three blocks per CU) or
 // 256x128 (two), 256 threads = 4 waves in 2x2, a stage of BK = 16 k = two
 // slabs of 8: global -> registers -> LDS, double-buffered, pipelined inside
 // one wave so the matrix core never waits on LDS (ordering fixed with
@@ -324,7 +325,9 @@ __global__ __launch_bounds__(kThreads, OCC) void gemm_f32_mfma(GemmArgs a) {
 // product is then taken as the six partial products
 //   a0 b2 + a1 b1 + a2 b0 + a0 b1 + a1 b0 + a0 b0
 // on v_mfma_f32_32x32x16_bf16, whose products are exact and whose sums are
-// fp32; what is left out (a1 b2, a2 b1, a2 b2) is below 2^-26 of the product.
+// fp32; what is left out (a1 b2, a2 b1, a2 b2) is at most 2^-24 of the product
+// (|a1| <= 2^-8, |a2| <= 2^-17 of a value) and 2^-27.5 of it in the root mean
+// square.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -475,11 +478,14 @@ struct SplitTile {
 };
 
 // Why: the fp32 MFMAs reach 151 TFLOP/s (0.96 of their peak) and bound every
-// large product.  Here 32768x6144x2048 (NT) takes 3.42 ms against 5.48, 241
-// TFLOP/s: matrix cores 75% busy while power holds the clock near 1.9 GHz (on
-// zeros, which cost little power, the same launch takes 2.64 ms).
-// Error against 64-bit sums, normal data, K = 256 / 2048 / 32768: 2.4e-7,
-// 7.0e-7, 3.0e-6 in the 2-norm, where fp32 MFMAs give 2.9e-7, 8.1e-7, 3.2e-6.
+// large product.  Here 32768x6144x2048 takes 3.7 ms in each layout against 5.5,
+// 222 TFLOP/s: matrix cores 70-74% busy while power holds the clock near 1.8
+// GHz (on zeros, which cost little power, the same launch takes 2.8 ms).
+// Error against 64-bit sums in the 2-norm, normal data, K = 32 / 256 / 2048:
+// 6.9e-8 / 2.4e-7 / 6.9e-7, where fp32 MFMAs give 1.0e-7 / 2.9e-7 / 8.1e-7; with
+// the 512-thread tile's segments 6.9e-8 / 1.7e-7 / 2.4e-7 (K = 32768: 3.1e-7
+// against 3.2e-6).  A sum of one term is rounded with 0.39 of a unit (rms)
+// instead of 0.29.
 //
 // The bf16 MFMAs round their sums very slightly downwards (a mean of -1.3e-7
 // of the mean magnitude at K = 2048, in proportion to the number of sums and
@@ -489,24 +495,28 @@ struct SplitTile {
 // sign flipped on the way to LDS, from 0.207 to 0.707 of K, which cancels the
 // bias of sums that stay the same size along K or grow as sqrt(K), and all
 // but 9% where they grow as K (nothing here depends on a row's or column's
-// place).  K splits start negated by the parity of the number's count of ones
-// (0 1 1 0 1 0 0 1 ...); the products of a batch all start alike.  Turning 256 accumulators costs about one stage.
+// place).  Two things it cannot balance: terms that all lie in one half of K (a
+// mean of 3e-8 at K = 2048, 6% of the spread) and a single pair of stages (K <=
+// 32: 1e-8).  K splits start negated by the parity of the number's count of
+// ones (0 1 1 0 1 0 0 1 ...); the products of a batch all start alike.  Turning
+// 256 accumulators costs about one stage.
 //
 // What the split cannot give: an infinity or NaN has no three parts, nor has a
 // value of 2^104 or more once scaled; such a result, or one past 2^80, is not
 // finite, which is found here, and it is taken again in fp32.
+//
 // The 512-thread tile has the registers for a second set of sums and adds up K
 // in segments of at most kSegK, an even number of them, with the same signs as
-// K splits: as exact as that many splits (1000x2048x2048 unsplit 4.85e-7 ->
-// 2.4e-7 in the 2-norm) without their planes.
+// K splits: as exact as that many splits (2048x1024x2048 in two chunks 4.85e-7
+// -> 2.4e-7 in the 2-norm) without their planes.
 constexpr int kSegK = 256;
 
 // THREADS = 256: 4 waves in 2x2, wave tiles (BM/2)x(BN/2); 512: 8 waves in
-// 4x2.  LDS is double buffered.  A 256x256 block has a CU to itself and one wave per SIMD, so the
-// order of the wave's own instructions is what keeps the matrix core busy:
-// it is written out MFMA by MFMA and pinned (sched_barrier), two to eight
-// VALU operations of the split between two MFMAs of 32 cycles each.  Left to
-// the compiler, the same work ran at 207 TFLOP/s instead of 241.
+// 4x2.  LDS is double buffered.  A 256x256 block has a CU to itself and one
+// wave per SIMD, so the order of the wave's own instructions is what keeps the
+// matrix core busy: it is written out MFMA by MFMA and pinned (sched_barrier),
+// two to eight VALU operations of the split between two MFMAs of 32 cycles
+// each.  Left to the compiler, the same work took 1.16 times as long.
 template <bool A_KC, bool B_KC, int BM, int BN, int THREADS, int OCC>
 __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   using TA = SplitTile<A_KC, BM, THREADS>;
@@ -1080,10 +1090,10 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
 // with 1 to 16 splits; choosing by them is on average 0.5% slower than the
 // best of those, at worst 4%.  The 512-thread tile is for grids of one block
 // per CU, where one wave per SIMD cannot issue fast enough (a stage alone
-// takes 0.37-0.44 us instead of 0.53: 256x576x576 13.2 -> 12.1 us,
-// 2048x576x1536 33.1 -> 29.7, 509x3072x1024 31.7 -> 28.6, 1000x2048x2048
-// 56.4 -> 52.4); with more blocks it is slower (4096x3072x1024 151 against
-// 130 us).
+// takes 0.37-0.44 us instead of 0.53: when it was added 256x576x576 went 13.2
+// -> 12.1 us, 2048x576x1536 33.1 -> 29.7, 509x3072x1024 31.7 -> 28.6,
+// 1000x2048x2048 56.4 -> 52.4); with more blocks it is slower (4096x3072x1024
+// 151 against 130 us).
 struct SplitPlan {
   int tile;         // index into kTiles
   int64_t splits;   // 1 = no K split
@@ -1294,8 +1304,9 @@ int gemm_run(int transa, int transb, int64_t M, int64_t N, int64_t K, float alph
         launch_reduce_n<8>,  launch_reduce_n<9>,  launch_reduce_n<10>, launch_reduce_n<11>,
         launch_reduce_n<12>, launch_reduce_n<13>, launch_reduce_n<14>, launch_reduce_n<15>,
         launch_reduce_n<16>};
-    kReduce[rvec ? std::min<int64_t>(splits, kMaxPlanes) : 0](blocks, static_cast<const float*>(workspace), C, M, N, ldc,
-                               static_cast<int>(splits), alpha, beta, rdyn, dyn_base, D, ldd, st);
+    kReduce[rvec ? std::min<int64_t>(splits, kMaxPlanes) : 0](
+        blocks, static_cast<const float*>(workspace), C, M, N, ldc, static_cast<int>(splits), alpha,
+        beta, rdyn, dyn_base, D, ldd, st);
     return launch_status();
   }
   if (fast) return launch_split(a, sp.tile, a_kc, b_kc, batch, st);

@@ -1,5 +1,5 @@
 #pragma once
-// Matrix multiply on the fp32 MFMA GEMM (mirrors ops/matmul.h of the reference).
+// Matrix multiply on the fp32 GEMM (mirrors ops/matmul.h of the reference).
 #include "ctd/tensor.h"
 
 namespace ctd::ops {

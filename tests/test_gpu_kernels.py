@@ -124,9 +124,9 @@ def gemm_ws(a, b, ta, tb, alpha=1.0, beta=0.0, c=None, ws_bytes=None):
                                      (1, 0, 5008), (0, 1, 5008)]
                          + [(ta, tb, K) for K in (1000, 2048) for ta in (0, 1) for tb in (0, 1)])
 def test_gemm_split_k_vs_oracle(ta, tb, K):
-    # Few output tiles: the K-split path with partials (K % 16 == 0 takes the
-    # LDS-DMA kernel, a ragged K the register-staged one), 16 splits of a long K
-    # and 3 or 8 of a short one.
+    # Few output tiles: the K-split path with partials (a K-contiguous operand of
+    # a ragged K takes the fp32 kernel), a long K in as many splits as the
+    # workspace holds and a short one.
     M, N = 132, 200
     r = rng(11 + 2 * ta + tb)
     a = r.standard_normal((K, M) if ta else (M, K)).astype(np.float32)
@@ -228,14 +228,14 @@ def test_gemm_split_k_weight_gradient_shape_vs_torch():
 
 @pytest.mark.parametrize("ta,tb,M,N,K", [
     (0, 1, 33000, 1000, 40), (0, 0, 33000, 1000, 40), (1, 0, 33000, 1000, 40),
-    (1, 1, 33000, 1000, 40),                        # register-staged kernel (K % 16 != 0)
+    (1, 1, 33000, 1000, 40),                        # a short first stage
     (0, 1, 33000, 1000, 48), (0, 0, 33000, 1000, 48), (1, 0, 33000, 1000, 48),
-    (1, 1, 33000, 1000, 48),                        # LDS-DMA kernel, M, N off the tile grid
-    (0, 1, 33001, 999, 48),                         # LDS-DMA, K-contiguous rows clamped
-    # one and two 16-k stages: the peeled k loop's DMA-free tail only
+    (1, 1, 33000, 1000, 48),                        # M, N off the tile grid
+    (0, 1, 33001, 999, 48),                         # K-contiguous rows past the operands
+    # one and two 16-k stages
     (0, 1, 33000, 1000, 16), (0, 0, 33000, 1000, 32), (1, 0, 33000, 1000, 16),
     (1, 1, 33000, 1000, 32), (0, 1, 500, 300, 16), (1, 0, 500, 300, 32),
-    (0, 1, 500, 300, 64),                           # 128x128 tiles, two stages of DMA ahead
+    (0, 1, 500, 300, 64),                           # 128x128 tiles, whole pairs of stages
 ])
 def test_gemm_large_tile_ragged_vs_oracle(ta, tb, M, N, K):
     # Enough tiles for the 256x128 kernels, with M and N off the tile grid.
@@ -683,11 +683,11 @@ def _gemm_ws(A, B, ta, tb, M, N, K, lda, ldb):
 
 
 @pytest.mark.parametrize("ta,tb,M,N,K", [
-    (0, 1, 4096, 2048, 512),    # Linear forward shape: 256x128 DMA tiles
-    (0, 1, 300, 200, 64),       # 128x128 DMA tiles, ragged edges
+    (0, 1, 4096, 2048, 512),    # Linear forward shape: large tiles
+    (0, 1, 300, 200, 64),       # 128x128 tiles, ragged edges
     (0, 0, 1000, 300, 48),      # NN
     (1, 0, 256, 128, 8192),     # TN with a K split: the reduce adds D
-    (1, 1, 200, 150, 70),       # K not whole 16-k stages: register-staged kernel
+    (1, 1, 200, 150, 70),       # rows that are not whole float4s: the fp32 kernel
     (0, 1, 5, 1000, 256),       # M <= 8: skinny kernel
     (0, 1, 100, 64, 0),         # K = 0: C = D
 ])
