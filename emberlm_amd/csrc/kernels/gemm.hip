@@ -10,8 +10,8 @@
 // 0.157.  Against 64-bit sums its error is 0.85 of theirs (see the kernel).
 //
 // Fallback, gemm_f32_mfma (rows that are not whole aligned float4s, offsets
-// past 2 GB, K of at most 8), whose tile also serves the split kernel's results
-// that are not finite: v_mfma_f32_32x32x2_f32, tiles 128x128 (three blocks per CU) or
+// past 2 GB), whose tile also serves the split kernel's results that are not
+// finite: v_mfma_f32_32x32x2_f32, tiles 128x128 (three blocks per CU) or
 // 256x128 (two), 256 threads = 4 waves in 2x2, a stage of BK = 16 k = two
 // slabs of 8: global -> registers -> LDS, double-buffered, pipelined inside
 // one wave so the matrix core never waits on LDS (ordering fixed with
@@ -484,8 +484,8 @@ struct SplitTile {
 // Error against 64-bit sums in the 2-norm, normal data, K = 32 / 256 / 2048:
 // 6.9e-8 / 2.4e-7 / 6.9e-7, where fp32 MFMAs give 1.0e-7 / 2.9e-7 / 8.1e-7; with
 // the 512-thread tile's segments 6.9e-8 / 1.7e-7 / 2.4e-7 (K = 32768: 3.1e-7
-// against 3.2e-6).  A sum of one term is rounded with 0.39 of a unit (rms)
-// instead of 0.29.
+// against 3.2e-6).  Only a sum of one or two terms that are not zero is further
+// off: one term is rounded with 0.39 of a unit (rms) instead of 0.29.
 //
 // The bf16 MFMAs round their sums very slightly downwards (a mean of -1.3e-7
 // of the mean magnitude at K = 2048, in proportion to the number of sums and
@@ -1203,16 +1203,13 @@ int launch_split(const GemmArgs& a, int tile, bool a_kc, bool b_kc, int64_t ny, 
                      : launch_split_tile<256, 256, 256, 1>(a, a_kc, b_kc, ny, st);
 }
 
-// How many of kTiles gemm_f32_split can use for these operands: none for a K of
-// at most 8, where the fp32 MFMAs, which round a lone product to nearest, are
-// closer to 64 bits when some terms are zero (K = 4 with one term: 2.5e-8
-// against 3.4e-8 in the 2-norm; from K = 12 with three terms on, further) and
-// the stores of C are what takes the time; none unless their rows are float4 rows that end on a whole float4; else those for which
+// How many of kTiles gemm_f32_split can use for these operands: none unless
+// their rows are float4 rows that end on a whole float4; else those for which
 // every byte offset inside a block's operand stage and output tile (the
 // tile's rows of a K-contiguous operand and of C, 16 k of the other) stays
 // below 2^31.
 int split_tiles(const GemmArgs& a, bool a_kc, bool b_kc, bool vec) {
-  if (a.K <= 8 || !vec || (a_kc ? a.K : a.M) % 4 != 0 || (b_kc ? a.K : a.N) % 4 != 0) return 0;
+  if (!vec || (a_kc ? a.K : a.M) % 4 != 0 || (b_kc ? a.K : a.N) % 4 != 0) return 0;
   const auto fits = [&](int64_t rows) {
     const int64_t top = (int64_t{1} << 29) - 1024;  // floats
     return (a_kc ? rows - 1 : 16) * a.lda < top && (b_kc ? rows - 1 : 16) * a.ldb < top &&

@@ -87,8 +87,8 @@ int ember_fill(float* p, int64_t n, float value, ember_stream_t s);
  * C[b] = alpha * op(A[b]) op(B[b]) + beta * C[b], fp32 operands and sums.  Each
  * value is split exactly into three bf16 values and a product is six bf16 MFMAs,
  * which omits at most 2^-24 of it; operands that the split kernel does not take
- * (rows that are not whole 16-byte pieces, or too far apart; K <= 8) and tiles
- * with results that are not finite run on the fp32 MFMAs.  Every finite value
+ * (rows that are not whole 16-byte pieces, or too far apart) and tiles with
+ * results that are not finite run on the fp32 MFMAs.  Every finite value
  * counts in full, subnormals included; what lies between the rows of an operand
  * does not reach C.
  * op(A) is MxK: A is stored [M,K] (lda >= K) or, when transa, [K,M] (lda >= M);
