@@ -268,7 +268,7 @@ Tensor linear_cross_entropy_masked(const Tensor& h, const Tensor& w, const Tenso
     if (want_h) dh = Tensor::empty({N, H}, DType::kFloat32, dev);
     if (want_w) dw = Tensor::empty({V, H}, DType::kFloat32, dev);  // running dlogits^T h
   }
-  // The active-row form needs the LDS-DMA GEMM's shapes: H, V in whole
+  // The active-row form needs the device-side-count GEMM's shapes: H, V in whole
   // 16-k stages, 16-byte aligned operands.
   const bool active_rows = g_head_active_rows.load() && N > 0 && H % 16 == 0 && V % 16 == 0 &&
                            reinterpret_cast<uintptr_t>(h.data_ptr()) % 16 == 0 &&

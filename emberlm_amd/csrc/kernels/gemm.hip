@@ -822,7 +822,8 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
             float out[V];
 #pragma unroll
             for (int c = 0; c < V; ++c) {
-              const float v = a.alpha * __builtin_fmaf(back, acc[i][j + c][e0 + e], 0.f);  // +0 for a zero
+              // + 0: a zero comes out positive
+              const float v = a.alpha * __builtin_fmaf(back, acc[i][j + c][e0 + e], 0.f);
               out[c] = kBeta ? v + a.beta * d[e][c] : v;
             }
             Out x;
