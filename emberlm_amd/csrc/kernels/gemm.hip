@@ -787,8 +787,9 @@ __global__ __launch_bounds__(THREADS, OCC) void gemm_f32_split(GemmArgs a) {
   const int lc = static_cast<int>(lrow * a.ldc * 4), ld = static_cast<int>(lrow * ldd * 4);
   // CHECKED: the wave tile reaches M.  BETA: the beta term is read, 16 values
   // before the first is used.  Where a lane has its FJ columns side by side (N
-  // is then whole float4s) they go in one access: 4 bytes at a time, 16 apart,
-  // were what a short K took its time for (8192x6144x32 TN 76 us).
+  // is then whole float4s) they go in one access, which may start at any float:
+  // 4 bytes at a time, 16 apart, were what a short K took its time for
+  // (8192x6144x32 TN 76 us, now 41).
   constexpr int V = B_KC || TB::P == 1 ? 1 : FJ;
   using Out = std::conditional_t<V == 4, u32x4, std::conditional_t<V == 2, u32x2, unsigned>>;
   static_assert(V == 1 || V == TB::P, "a lane's columns");

@@ -1057,6 +1057,31 @@ def test_gemm_ragged_k_takes_no_longer_than_the_next_whole_one(tb):
     assert best[0] <= 1.2 * best[1], best
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(140, 132, 52), (1000, 2052, 64), (4092, 2052, 96),
+                                   (8196, 2564, 64)])
+@pytest.mark.parametrize("off,pad", [(1, 3), (2, 2), (3, 1)])
+def test_gemm_output_and_addend_of_any_alignment(ta, tb, M, N, K, off, pad):
+    """C and D that start `off` floats past a 16-byte line with rows `pad` past whole float4s:
+    the bits of the aligned call, and nothing written between the rows."""
+    g = torch.Generator(device="cuda").manual_seed(M + off)
+    A = torch.randn((K, M) if ta else (M, K), device="cuda", generator=g)
+    B = torch.randn((N, K) if tb else (K, N), device="cuda", generator=g)
+    D = torch.randn(M, N, device="cuda", generator=g)
+    ld = N + pad + (-N) % 4
+    Dm = torch.zeros(M * ld + off, device="cuda")[off:].view(M, ld)
+    Dm[:, :N] = D
+    want = empty((M, N))
+    args = (ta, tb, M, N, K, 1.0, p(A), A.shape[1], p(B), B.shape[1])
+    call("ember_gemm_f32_add", *args, p(D), N, p(want), N, None, 0, None)
+    C1 = torch.full((M * ld + off,), 7.0, device="cuda")[off:].view(M, ld)
+    call("ember_gemm_f32_add", *args, p(Dm), ld, p(C1), ld, None, 0, None)
+    assert torch.equal(C1[:, :N], want) and (C1[:, N:] == 7.0).all()
+    call("ember_gemm_f32", ta, tb, M, N, K, 1.0, p(A), A.shape[1], 0, p(B), B.shape[1], 0, 0.0,
+         p(C1), ld, 0, 1, None)
+    assert torch.equal(C1[:, :N] + D, want) and (C1[:, N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dim,ta,tb", [(0, 0, 1), (1, 1, 0)])
 def test_gemm_dyn_on_rows_too_long_for_the_split_kernel(dim, ta, tb):
     """A device-side count on the fp32 kernel, which takes rows past 2 GB of offsets."""
